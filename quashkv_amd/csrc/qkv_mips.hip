@@ -1,5 +1,6 @@
-// Maximum inner-product search over K rows (QuashIndex.search): query operands
-// from prepare_mfma, integer-MFMA scoring, streaming top-k.
+// Maximum inner-product search over K rows (QuashIndex.search): a one-digit
+// filter with rigorous bounds and exact scores of what passes it, or a full scan
+// with streaming top-k; query operands from prepare_mfma.
 #include <math.h>
 
 #include <algorithm>
@@ -62,7 +63,8 @@ __global__ __launch_bounds__(256, 2) void mips_scan(const qkv_v4i* __restrict__ 
                                                  int nvc, int64_t vlen, int64_t n_items, int k,
                                                  float* __restrict__ cand_s,
                                                  int* __restrict__ cand_i,
-                                                 uint32_t* __restrict__ gth) {
+                                                 uint32_t* __restrict__ gth,
+                                                 const int* __restrict__ over, int cap) {
   using C = MipsCfg<MB, PDW>;
   constexpr int NU = C::NU, QC = C::QC, RAWD = C::RAWD;
   constexpr int QW = 4 * QC;                      // queries per wave
@@ -118,6 +120,10 @@ __global__ __launch_bounds__(256, 2) void mips_scan(const qkv_v4i* __restrict__ 
   for (int64_t item = blockIdx.x; item < n_items; item += gridDim.x) {
     const int vc = static_cast<int>(item / qtiles), qt = static_cast<int>(item % qtiles);
     const int chunk0 = (qt * 4 + wave) * QC;  // first query chunk of this wave
+    if (over != nullptr) {  // behind the filter: only tiles with an overflowed query
+      const int qo = qt * 4 * QW + tid;
+      if (!__syncthreads_or(tid < 4 * QW && qo < M && over[qo] > cap)) continue;
+    }
     const int64_t v0 = int64_t(vc) * vlen;
     const int64_t v1 = min<int64_t>(N, v0 + vlen);
 
@@ -298,9 +304,11 @@ __global__ __launch_bounds__(256, 2) void mips_scan(const qkv_v4i* __restrict__ 
 __global__ __launch_bounds__(64) void mips_merge(const float* __restrict__ cand_s,
                                                  const int* __restrict__ cand_i, int nsplit,
                                                  int k, float* __restrict__ out_s,
-                                                 int64_t* __restrict__ out_i) {
+                                                 int64_t* __restrict__ out_i,
+                                                 const int* __restrict__ over, int cap) {
   extern __shared__ __align__(16) float smem_mm[];
   const int q = blockIdx.x, lane = threadIdx.x;
+  if (over != nullptr && over[q] <= cap) return;
   const int n = nsplit * k;
   float* cs = smem_mm;
   int* ci = reinterpret_cast<int*>(smem_mm + n);
@@ -340,6 +348,634 @@ __global__ __launch_bounds__(64) void mips_merge(const float* __restrict__ cand_
   }
 }
 
+
+// ------------------------------------------------------------ filtered search
+//
+// The full scan above spends 4 query digits on every plane bit of every vector;
+// only the handful of scores near the top need them.  Here a coordinate's code
+// becomes one small integer L[code] (LUT, c[code] ~ a L[code]) and its weight
+// q~_j one int8 digit, the QJL bit likewise, so that
+//   score / n = f I - sum_j w_j + e,   I = sum_j d_j L[code_j] + dq_j V b_j
+// exactly in int32, with |e| bounded from the digits' residuals (about 0.13
+// standard deviations of the scores).  So:
+//   1. mips_pass<false> takes the lower bounds of every 8th 16-vector group and
+//      keeps the largest one of each (stream, column): maxima of disjoint sets
+//      of vectors, so mips_bound's k-th largest of them bounds the k-th best
+//      score from below;
+//   2. mips_pass<true> lists the vectors whose upper bound reaches that bound
+//      (about 25 k per query on N(0, 1) data): every vector of the exact top k,
+//      ties included, is among them;
+//   3. mips_pick scores the listed vectors with all four digits, the same
+//      integers and float operations as the full scan, and takes the k best.
+// A query whose list overflows, or whose weights are not finite or all zero,
+// goes to the full scan.  The results are the full scan's bit for bit.
+//
+// Measured (10^6 vectors, 10^4 queries, d = 128, 3 bits, top-10): 3.02 ms against
+// the full scan's 13.1: pass 2 ~2.4 ms (matrix cores busy ~45 %; MFMA time 1.06
+// ms), pass 1 0.3, the exact scores 0.19.  QT = 4 / 6 / 8: 3.98 / 3.22 / 3.02 ms.
+// Six bit-plane operands in place of the level bytes (one digit, band twice as
+// wide, 24 MFMAs per 64 queries) left half of the lists past their cap.
+//
+// Bounds: int8 MFMA, d / 32 per 16 queries x 16 vectors (the full scan at 2 MSE
+// bits, d = 128: 24), beside ~41 VALU instructions of expansion per 16 vectors
+// and one compare per score.  A wave holds the operands of 16 QT queries in
+// registers and streams 16-vector groups from L2 into registers two groups
+// ahead; no barrier, so the waves drift apart and one's VALU overlaps another's
+// MFMAs.
+constexpr int kNoI = -(1 << 30);   // no value of I (|I| < 2^22) brings it to 0
+constexpr int kFiltStep = 8;       // groups per sampled group of pass 1, from
+constexpr int64_t kFiltStepN = 8192;     // this many vectors (below, pass 1 takes every group)
+constexpr int kFiltQueue = 64;     // candidates a wave holds in LDS before a flush
+constexpr int kFiltQT = 8;         // 16-query tiles per wave, many queries
+constexpr int kFiltKMax = 64;      // k up to which the filter runs
+constexpr int64_t kFiltMinN = 256;  // vectors from which the filter runs
+
+// The codebook's integer levels: c[code] = a L[code] + (at most delta), L as the
+// bytes of (hi, lo); the QJL bit's byte value V = 1 << vlog, 2 qjl_scale <= a V.
+struct FiltTab {
+  uint32_t lo, hi;
+  float a, delta;
+  int lmax, vlog;
+};
+
+// Lane group g expands word g of each plane (d = 128; d = 96: group 3 has none)
+// into NU = 4 operands, MSE bits 0-3 and 4-7 of each byte, then the QJL bits; at
+// d = 64 word g % 2, the bits 4 (g / 2) .. + 3 of each byte, NU = 2.
+template <int PDW>
+struct FiltCfg {
+  static constexpr int NU = PDW == 2 ? 2 : 4;
+};
+
+// Filter operands of one 16-query tile per workgroup, from q~ and w =
+// alpha |q~| S (prepare_mfma's qw): 16 threads per query, d / 16 coordinates
+// each.  ciu / cil: the bounds' constants in units of f, rounded outwards.  The
+// slack covers the rounding of the exact path's 30-bit weights (at most 64 2^-fq
+// for each of 640) and of its floats.
+template <int PDW>
+__global__ __launch_bounds__(256) void mips_fprep(const float* __restrict__ qw,
+                                                  const float* __restrict__ rowc, int M,
+                                                  FiltTab ft, uint32_t* __restrict__ af,
+                                                  int* __restrict__ ciu, int* __restrict__ cil,
+                                                  int* __restrict__ cnt, int cap) {
+  constexpr int NU = FiltCfg<PDW>::NU, NWD = NU * 256;
+  constexpr int JT = PDW * 2;  // coordinates per thread
+  __shared__ uint32_t img[NWD];
+  int8_t* ib = reinterpret_cast<int8_t*>(img);
+  const int tid = threadIdx.x, m = tid >> 4, t16 = tid & 15;
+  for (int i = tid; i < NWD; i += 256) img[i] = 0;
+  const int q = blockIdx.x * 16 + m, qc = min(q, M - 1);
+  float v[JT], w[JT];
+  float mx = 0.f, l1 = 0.f, sw = 0.f, aw = 0.f;
+#pragma unroll
+  for (int x = 0; x < JT; ++x) {
+    const int j = t16 + 16 * x;
+    v[x] = qw[int64_t(qc) * 256 + j];
+    w[x] = qw[int64_t(qc) * 256 + 128 + j];
+    mx = fmaxf(mx, fabsf(v[x]));
+    l1 += fabsf(v[x]);
+    sw += w[x];
+    aw += fabsf(w[x]);
+  }
+#pragma unroll
+  for (int o = 8; o > 0; o >>= 1) {
+    mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+    l1 += __shfl_xor(l1, o, 64);
+    sw += __shfl_xor(sw, o, 64);
+    aw += __shfl_xor(aw, o, 64);
+  }
+  const float f = mx * ft.a / 127.f;
+  const bool ok = f > 1e-30f && l1 < 1e30f && aw < 1e30f;  // false for NaN sums too
+  const float rf = ok ? 1.f / f : 0.f;
+  const float iv = 1.f / static_cast<float>(1 << ft.vlog);
+  __syncthreads();
+  float er = 0.f, eu = 0.f, el = 0.f;
+  // byte of operand dword e of MFMA u, lane group g: (word wd, bit i of byte beta)
+  auto byte_at = [&](int j, bool qjl) {
+    const int wd = j >> 5, i = j & 7, beta = (j >> 3) & 3;
+    int g, u;
+    if constexpr (PDW == 2) {
+      g = wd + 2 * (i >> 2);
+      u = qjl ? 1 : 0;
+    } else {
+      g = wd;
+      u = (qjl ? 2 : 0) + (i >> 2);
+    }
+    return ((u * 64 + m + 16 * g) * 4 + (i & 3)) * 4 + beta;
+  };
+  auto digit = [&](float W, int at, float& r) {
+    const float d = fminf(fmaxf(rintf(W * rf), -127.f), 127.f);
+    r = fmaf(-d, f, W);
+    ib[at] = ok ? static_cast<int8_t>(static_cast<int>(d)) : 0;
+  };
+#pragma unroll
+  for (int x = 0; x < JT; ++x) {
+    const int j = t16 + 16 * x;
+    float r;
+    digit(v[x] * ft.a, byte_at(j, false), r);
+    er += fabsf(r);
+    digit(2.f * w[x] * iv, byte_at(j, true), r);
+    eu += fmaxf(r, 0.f);
+    el += fmaxf(-r, 0.f);
+  }
+#pragma unroll
+  for (int o = 8; o > 0; o >>= 1) {
+    er += __shfl_xor(er, o, 64);
+    eu += __shfl_xor(eu, o, 64);
+    el += __shfl_xor(el, o, 64);
+  }
+  if (t16 == 0) {
+    const float cr = rowc[int64_t(qc) * 2];
+    const float vq = static_cast<float>(1 << ft.vlog);
+    const float slack = 1.9e-6f * (2.f * ft.a * ft.lmax * l1 + 4.f * aw + fabsf(cr)) +
+                        65536.f * rowc[int64_t(qc) * 2 + 1];
+    const float e = er * ft.lmax + ft.delta * l1 + slack;
+    const bool use = ok && fabsf(cr) < 1e30f;
+    ciu[q] = use ? static_cast<int>(ceilf((e + vq * eu - sw) * rf)) + 1 : 0;
+    cil[q] = use ? static_cast<int>(floorf((-e - vq * el - sw) * rf)) - 1 : 0;
+    cnt[q] = use || q >= M ? 0 : cap + 1;  // past cap: left to the full scan
+  }
+  __syncthreads();
+  for (int i = tid; i < NWD; i += 256) af[int64_t(blockIdx.x) * NWD + i] = img[i];
+}
+
+// One pass over the database.  Waves: (query tile of 16 QT, stream p of P);
+// stream p takes the groups p, p + P, ... of the ng (sampled: every gstep-th)
+// 16-vector groups, so that all waves sweep the database together, and with P a
+// multiple of 8 a stream's waves share an XCD's L2.
+//
+// While a group's norms all lie within 0.1 % below nq (an L2-normalised
+// database), the scores are compared as integers: COLLECT starts the
+// accumulators at minus the queries' thresholds at nq, so that a set sign bit in
+// every accumulator (one AND of two values each) dismisses the group, and the
+// sampling pass keeps integer maxima.  Other groups take the float products.
+// Such a group costs 4 QT MFMAs (512 cycles at QT = 8) and ~75 VALU
+// instructions; the next group's expansion and the reductions are scheduled
+// between the MFMAs (three VALU instructions fill an MFMA's 16 cycles).
+template <int MB, int PDW, int QT, bool COLLECT>
+__global__ __launch_bounds__(256, 2) void mips_pass(
+    const qkv_v4i* __restrict__ af, const int* __restrict__ cinit, const float* __restrict__ thr,
+    const uint8_t* __restrict__ kst, const float* __restrict__ norms, int64_t N, int ntile,
+    int wq, int pb, int64_t ng, int gstep, FiltTab ft, float* __restrict__ mxo,
+    int* __restrict__ cnt, int* __restrict__ cand, int cap) {
+  constexpr int NU = FiltCfg<PDW>::NU, RAWD = (MB + 1) * PDW, NP = MB + 1;
+  constexpr int NI = PDW == 2 ? 4 : 8;  // bits of each byte a lane expands
+  constexpr int kQ = COLLECT ? kFiltQueue + 256 * QT : 1;  // one group lists 256 QT at most
+  __shared__ int qv[COLLECT ? 4 : 1][kQ];
+  __shared__ uint8_t qq[COLLECT ? 4 : 1][kQ];
+  __shared__ __align__(16) int cis[4][16 * QT];
+  __shared__ __align__(16) float ths[COLLECT ? 4 : 1][COLLECT ? 16 * QT : 4];
+  __shared__ float mxl[COLLECT ? 1 : 4][COLLECT ? 1 : 4 * QT][64];  // running maxima
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int ln = lane & 15, lg = lane >> 4;
+  const int ws = 4 / wq;  // streams per workgroup
+  const int tile = (blockIdx.x / pb) * wq + wave % wq;
+  const int p = (blockIdx.x % pb) * ws + wave / wq, P = pb * ws;
+  if (tile >= ntile) return;  // (no barrier below: the LDS arrays are each wave's own)
+
+  qkv_v4i a[QT][NU];
+#pragma unroll
+  for (int t = 0; t < QT; ++t)
+#pragma unroll
+    for (int u = 0; u < NU; ++u)
+      a[t][u] = af[((int64_t(tile) * QT + t) * NU + u) * 64 + lane];
+  for (int i = lane; i < 16 * QT; i += 64) {
+    cis[wave][i] = cinit[int64_t(tile) * 16 * QT + i];
+    if constexpr (COLLECT) ths[wave][i] = thr[int64_t(tile) * 16 * QT + i];
+  }
+  // COLLECT: minus the integer thresholds at nq; else the largest I at nq
+  qkv_v4i ti[COLLECT ? QT : 1];
+  int mi[COLLECT ? 1 : 4 * QT];
+  float nq = -1.f;
+  if constexpr (!COLLECT) {
+#pragma unroll
+    for (int t = 0; t < 4 * QT; ++t) mxl[wave][t][lane] = -INFINITY;
+  }
+  if constexpr (!COLLECT) {
+#pragma unroll
+    for (int t = 0; t < 4 * QT; ++t) mi[t] = kNoI;
+  }
+
+  struct Row {
+    uint32_t w[NP];
+    float n;
+  };
+  // this lane's word of each plane: 32-bit lane offsets from a wave-uniform base
+  const uint32_t wo = PDW == 2 ? (lg & 1) : PDW == 3 ? min(lg, 2) : lg;
+  auto load = [&](int64_t x) {
+    Row r;
+    const int64_t v0 = min<int64_t>(x, ng - 1) * gstep * 16;
+    // (the last group may be partial; no branch, which would split the schedule)
+    const uint32_t left = static_cast<uint32_t>(min<int64_t>(N - 1 - v0, 15));
+    const uint32_t ni = min<uint32_t>(ln, left), lo = (ni * RAWD + wo) * 4;
+    const uint8_t* base = kst + v0 * (RAWD * 4);
+#pragma unroll
+    for (int j = 0; j < NP; ++j)
+      r.w[j] = *reinterpret_cast<const uint32_t*>(base + (lo + 4 * PDW * j));
+    const float n = norms[v0 + ni];
+    // past the end (and, among the lower bounds, a negative norm): passes no compare
+    r.n = ni == static_cast<uint32_t>(ln) && (COLLECT || n >= 0.f) ? n : __builtin_nanf("");
+    return r;
+  };
+
+  // the NU operands of 16 vectors: codes' levels, then QJL bits (byte value V)
+  const uint32_t vmask = 0x01010101u << ft.vlog;
+  auto expand = [&](const Row& row, qkv_v4i* bo) {
+    uint32_t w[NP];
+#pragma unroll
+    for (int j = 0; j < NP; ++j) w[j] = PDW == 2 ? row.w[j] >> (4 * (lg >> 1)) : row.w[j];
+    // codes of the even and of the odd bits, two bits each (their low two bits)
+    uint32_t ze, zo;
+    if constexpr (MB == 1) {
+      ze = w[0];
+      zo = w[0] >> 1;
+    } else {
+      ze = (w[0] & 0x55555555u) | ((w[1] << 1) & 0xaaaaaaaau);
+      zo = ((w[0] >> 1) & 0x55555555u) | (w[1] & 0xaaaaaaaau);
+    }
+    const uint32_t y = __builtin_amdgcn_alignbit(w[MB], w[MB], 32 - ft.vlog);  // left by vlog
+    constexpr uint32_t zm = MB == 1 ? 0x01010101u : 0x03030303u;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      uint32_t sel = ((i & 1 ? zo : ze) >> (i & ~1)) & zm;
+      if constexpr (MB == 3)
+        sel |= (i < 2 ? w[2] << (2 - i) : w[2] >> (i - 2)) & 0x04040404u;
+      bo[i >> 2][i & 3] = static_cast<int>(__builtin_amdgcn_perm(ft.hi, ft.lo, sel));
+      bo[NU / 2 + (i >> 2)][i & 3] = static_cast<int>(__builtin_amdgcn_alignbit(y, y, i) & vmask);
+    }
+  };
+
+  int qn = 0;  // queued candidates (wave-uniform)
+  auto flush = [&]() {
+    bool any = false;
+    for (int i = lane; i < qn; i += 64) {
+      const int ql = qq[wave][i];
+      const int64_t q = int64_t(tile) * 16 * QT + ql;
+      const int at = atomicAdd(&cnt[q], 1);
+      if (at < cap) {
+        cand[q * cap + at] = qv[wave][i];
+      } else {  // the query goes to the full scan: take no more of it
+        ths[wave][ql] = __builtin_nanf("");
+        any = true;
+      }
+    }
+    qn = 0;
+    if (__builtin_amdgcn_ballot_w64(any)) nq = -1.f;  // (new integer thresholds)
+  };
+
+  // COLLECT: minus the smallest I that may pass at norms in (0.999 nq, nq]
+  auto thresholds = [&]() {
+    const float rhi = 1.f / nq, rlo = rhi * 1.00101f;
+#pragma unroll
+    for (int t = 0; t < QT; ++t) {
+      const qkv_v4f th = *reinterpret_cast<const qkv_v4f*>(&ths[wave][16 * t + 4 * lg]);
+      const qkv_v4i ci = *reinterpret_cast<const qkv_v4i*>(&cis[wave][16 * t + 4 * lg]);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float x = fminf(th[r] * rhi, th[r] * rlo);
+        const float y = x - fabsf(x) * 1e-6f;
+        ti[t][r] = th[r] == th[r] ? ci[r] - static_cast<int>(floorf(fminf(fmaxf(y, -1e9f), 1e9f)))
+                                  : kNoI;
+      }
+    }
+  };
+  // sampling: the integer maxima at nq into the float ones
+  auto settle_max = [&]() {
+#pragma unroll
+    for (int t = 0; t < QT; ++t) {
+      const qkv_v4i ci = *reinterpret_cast<const qkv_v4i*>(&cis[wave][16 * t + 4 * lg]);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        if (mi[4 * t + r] > kNoI) {
+          const float s = static_cast<float>(mi[4 * t + r] + ci[r]) * nq;
+          float& m = mxl[wave][4 * t + r][lane];
+          m = fmaxf(m, s >= 0.f ? 0.998999f * s : s);
+        }
+        mi[4 * t + r] = kNoI;
+      }
+    }
+  };
+  auto product = [&](int t, const qkv_v4i* bo, qkv_v4i c) {
+#pragma unroll
+    for (int u = 0; u < NU; ++u) c = mfma_i8(a[t][u], bo[u], c);
+    return c;
+  };
+  auto push = [&](uint64_t h, int ql, int64_t x) {
+    const int nh = __builtin_popcountll(h);
+    if ((h >> lane) & 1u) {
+      const int at = qn + __builtin_popcountll(h & ((uint64_t(1) << lane) - 1));
+      qv[wave][at] = static_cast<int>(x * 16 + ln);
+      qq[wave][at] = static_cast<uint8_t>(ql + 4 * lg);
+    }
+    qn += nh;
+  };
+
+  // group x from its operands cur and norms nc, while row (the group P on)
+  // becomes nxt and the row's registers take the load of the group 3 P on
+  auto body = [&](const qkv_v4i* cur, float nc, qkv_v4i* nxt, float& nn, Row& row, int64_t x) {
+    bool uni = __builtin_amdgcn_ballot_w64(nc <= nq && nc > nq * 0.999f) == ~0ull;
+    if (!uni) {
+      // the largest norm, its low 12 mantissa bits rounded up: the next nq
+      float m = nc == nc ? nc : 0.f;
+#pragma unroll
+      for (int o = 8; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+      const float c = __uint_as_float((__float_as_uint(m) + 0xfffu) & ~0xfffu);
+      if (__builtin_amdgcn_ballot_w64(nc <= c && nc > c * 0.999f) == ~0ull && c > 1e-30f &&
+          c < 1e30f) {
+        if constexpr (!COLLECT) settle_max();
+        nq = c;
+        if constexpr (COLLECT) thresholds();
+        uni = true;
+      }
+    }
+    if (uni) {
+      int m[QT];
+#pragma unroll
+      for (int t = 0; t < QT; t += 2) {  // two independent accumulator chains
+        qkv_v4i c0 = {0, 0, 0, 0}, c1 = {0, 0, 0, 0};
+        if constexpr (COLLECT) {
+          c0 = ti[t];
+          if (t + 1 < QT) c1 = ti[t + 1];
+        }
+#pragma unroll
+        for (int u = 0; u < NU; ++u) {
+          c0 = mfma_i8(a[t][u], cur[u], c0);
+          if (t + 1 < QT) c1 = mfma_i8(a[t + 1 < QT ? t + 1 : 0][u], cur[u], c1);
+        }
+        if constexpr (COLLECT) {
+          m[t] = c0[0] & c0[1] & c0[2] & c0[3];
+          if (t + 1 < QT) m[t + 1] = c1[0] & c1[1] & c1[2] & c1[3];
+        } else {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            mi[4 * t + r] = max(mi[4 * t + r], c0[r]);
+            if (t + 1 < QT) mi[4 * t + 4 + r] = max(mi[4 * t + 4 + r], c1[r]);
+          }
+        }
+      }
+      expand(row, nxt);
+#pragma unroll
+      for (int u = 0; u < NU; ++u) asm volatile("" : "+v"(nxt[u]));  // (not sunk past the branch)
+      nn = row.n;
+      row = load(x + 3 * P);
+#pragma unroll
+      for (int i = 0; i < QT * NU; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);   // MFMA
+        __builtin_amdgcn_sched_group_barrier(0x2, 2, 0);   // VALU
+      }
+      if constexpr (COLLECT) {
+        int all = m[0];
+#pragma unroll
+        for (int t = 1; t < QT; ++t) all &= m[t];
+        if (__builtin_amdgcn_ballot_w64(all >= 0)) {
+#pragma unroll
+          for (int t = 0; t < QT; ++t) {
+            if (__builtin_amdgcn_ballot_w64(m[t] >= 0) == 0) continue;
+            const qkv_v4i c = product(t, cur, ti[t]);  // again: the sums were not kept
+            mfma_settle();
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              const uint64_t h = __builtin_amdgcn_ballot_w64(c[r] >= 0);
+              if (h) push(h, 16 * t + r, x);
+            }
+          }
+          if (qn > kFiltQueue) flush();
+        }
+      }
+      return;
+    }
+#pragma unroll
+    for (int t = 0; t < QT; ++t) {
+      const qkv_v4i c = product(t, cur, qkv_v4i{0, 0, 0, 0});
+      const qkv_v4i ci = *reinterpret_cast<const qkv_v4i*>(&cis[wave][16 * t + 4 * lg]);
+      mfma_settle();
+      if constexpr (COLLECT) {
+        const qkv_v4f th = *reinterpret_cast<const qkv_v4f*>(&ths[wave][16 * t + 4 * lg]);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          // (the bounds hold for norms >= 0: any other vector is listed)
+          const uint64_t h = __builtin_amdgcn_ballot_w64(
+              static_cast<float>(c[r] + ci[r]) * nc >= th[r] || (nc < 0.f && th[r] == th[r]));
+          if (h) push(h, 16 * t + r, x);
+        }
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          float& m = mxl[wave][4 * t + r][lane];
+          m = fmaxf(m, static_cast<float>(c[r] + ci[r]) * nc);
+        }
+      }
+    }
+    if constexpr (COLLECT) {
+      if (qn > kFiltQueue) flush();
+    }
+    // (opaque: kept apart from the same lines above, whose place is among the MFMAs)
+#pragma unroll
+    for (int j = 0; j < NP; ++j) asm volatile("" : "+v"(row.w[j]));
+    expand(row, nxt);
+    nn = row.n;
+    row = load(x + 3 * P);
+  };
+
+  qkv_v4i b0[NU], b1[NU];
+  float n0, n1 = 0.f;
+  Row r1 = load(p), r0 = load(int64_t(p) + P);
+  expand(r1, b0);
+  n0 = r1.n;
+  r1 = load(int64_t(p) + 2 * P);
+  for (int64_t x = p; x < ng; x += 2 * P) {
+    body(b0, n0, b1, n1, r0, x);
+    if (x + P < ng) body(b1, n1, b0, n0, r1, x + P);
+  }
+  if constexpr (COLLECT) {
+    flush();
+  } else {
+    settle_max();
+#pragma unroll
+    for (int t = 0; t < QT; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int64_t q = (int64_t(tile) * QT + t) * 16 + 4 * lg + r;
+        mxo[(q * P + p) * 16 + ln] = mxl[wave][4 * t + r][lane];
+      }
+  }
+}
+
+// Threshold of one query per workgroup: the k-th largest of 256 R maxima, each
+// the largest of a disjoint share of the query's n stream maxima, lowered by the
+// rounding of one float product.  NaN (admits nothing) for a query the filter
+// does not serve: past the cap already, or without k finite maxima.
+template <int R>
+__global__ __launch_bounds__(256) void mips_bound(const float* __restrict__ mx, int n, int k,
+                                                  int M, float* __restrict__ thr,
+                                                  int* __restrict__ cnt, int cap) {
+  __shared__ float sh[256 * R];
+  const int q = blockIdx.x, tid = threadIdx.x;
+  if (q >= M || cnt[q] > cap) {
+    if (tid == 0) thr[q] = __builtin_nanf("");
+    return;
+  }
+#pragma unroll
+  for (int x = 0; x < R; ++x) {
+    float m = -INFINITY;
+#pragma unroll 4
+    for (int i = tid + 256 * x; i < n; i += 256 * R) m = fmaxf(m, mx[int64_t(q) * n + i]);
+    sh[tid + 256 * x] = m;
+  }
+  __syncthreads();
+  if (tid >= 64) return;
+  float v[4 * R];
+#pragma unroll
+  for (int x = 0; x < 4 * R; ++x) v[x] = sh[tid + 64 * x];
+  float kth = -INFINITY;
+  for (int r = 0; r < k; ++r) {
+    float best = v[0];
+#pragma unroll
+    for (int x = 1; x < 4 * R; ++x) best = fmaxf(best, v[x]);
+    kth = wave_max_dpp(best);
+    const uint64_t who = __builtin_amdgcn_ballot_w64(best == kth);
+    if (tid == static_cast<int>(__builtin_ctzll(who))) {
+      bool out = false;  // the first slot that holds it
+#pragma unroll
+      for (int x = 0; x < 4 * R; ++x)
+        if (!out && v[x] == kth) {
+          v[x] = -INFINITY;
+          out = true;
+        }
+    }
+  }
+  if (tid == 0) {
+    const bool ok = fabsf(kth) < INFINITY;  // else: left to the full scan
+    thr[q] = ok ? kth - fabsf(kth) * 1.9e-6f : __builtin_nanf("");
+    if (!ok) cnt[q] = cap + 1;
+  }
+}
+
+// Exact scores of a query's listed vectors (the full scan's integers: digit
+// pairs of each weight, summed over the set plane bits) and the k best of them
+// (score descending, index ascending).  One query per workgroup, a thread per
+// vector; the query's weights as LDS tables that all lanes read together.
+template <int MB, int PDW>
+__global__ __launch_bounds__(256) void mips_pick(const qkv_v4i* __restrict__ aq,
+                                                 const float* __restrict__ rowc,
+                                                 const uint8_t* __restrict__ kst,
+                                                 const float* __restrict__ norms, int k,
+                                                 const int* __restrict__ cnt,
+                                                 const int* __restrict__ cand, int cap,
+                                                 float* __restrict__ out_s,
+                                                 int64_t* __restrict__ out_i) {
+  using F = MipsCfg<MB, PDW>;
+  constexpr int NPL = F::NPL, NU = F::NU, DPL = F::DPL, RAWD = F::RAWD;
+  constexpr int VD = NPL * PDW;  // virtual row dwords
+  constexpr bool kPair = NU * (1 << 20) < (1 << 23);  // two exact halves, as the full scan
+  __shared__ int tab[VD * 32][kPair ? 2 : 4];
+  extern __shared__ __align__(16) float smem_mk[];  // [cap] scores, [cap] indices
+  const int q = blockIdx.x, tid = threadIdx.x;
+  const int n = cnt[q];
+  if (n > cap) return;
+  float* cs = smem_mk;
+  int* ci = reinterpret_cast<int*>(smem_mk + cap);
+  // digit v of the weight at virtual bit (plane, coordinate) from the operand image
+  const int8_t* ab = reinterpret_cast<const int8_t*>(aq) + int64_t(q >> 2) * NU * 1024;
+  for (int p = tid; p < VD * 32; p += 256) {
+    const int pl = p / (32 * PDW), j = p - pl * 32 * PDW;
+    const int w32 = pl * 4 + (j >> 5), i = p & 7, e = i & 3, beta = (p >> 3) & 3;
+    const int g = w32 / DPL, u = 2 * (w32 - g * DPL) + (i >> 2);
+    const int8_t* src = ab + ((u * 64 + 16 * g + 4 * (q & 3)) * 4 + e) * 4 + beta;
+    const int m = i == 7 ? -128 : 1 << i;
+    const int d0 = src[0], d1 = src[16], d2 = src[32], d3 = src[48];
+    if constexpr (kPair) {
+      tab[p][0] = m * (d0 + 256 * d1);
+      tab[p][1] = m * (d2 + 256 * d3);
+    } else {
+      tab[p][0] = m * d0;
+      tab[p][1] = m * d1;
+      tab[p][2] = m * d2;
+      tab[p][3] = m * d3;
+    }
+  }
+  const float cr = rowc[int64_t(q) * 2], fq = rowc[int64_t(q) * 2 + 1];
+  __syncthreads();
+  for (int c = tid; c < n; c += 256) {
+    const int v = cand[int64_t(q) * cap + c];
+    const uint32_t* src = reinterpret_cast<const uint32_t*>(kst) + int64_t(v) * RAWD;
+    int z[kPair ? 2 : 4] = {};
+    // (rolled: unrolled, the tables move out of the candidate loop into registers)
+#pragma unroll 1
+    for (int wd = 0; wd < VD; ++wd) {
+      uint32_t x;
+      if constexpr (MB <= 2) {
+        x = src[wd];
+      } else {  // virtual planes b0, b1, b2, their parity, QJL
+        x = src[wd < 3 * PDW ? wd : wd - PDW];
+        if (wd >= 3 * PDW && wd < 4 * PDW) x ^= src[wd - 3 * PDW] ^ src[wd - 2 * PDW];
+      }
+      const int* tp = tab[wd * 32];
+#pragma unroll
+      for (int b = 0; b < 32; ++b) {
+        const int on = -static_cast<int>((x >> b) & 1u);
+#pragma unroll
+        for (int h = 0; h < (kPair ? 2 : 4); ++h) z[h] += tp[b * (kPair ? 2 : 4) + h] & on;
+      }
+    }
+    const float nv = norms[v];
+    float s;
+    if constexpr (kPair) {
+      s = nv * fmaf(static_cast<float>(z[1]), 65536.f * fq,
+                    fmaf(static_cast<float>(z[0]), fq, cr));
+    } else {
+      const float zz = static_cast<float>(z[0]) + 256.f * static_cast<float>(z[1]) +
+                       65536.f * static_cast<float>(z[2]) + 16777216.f * static_cast<float>(z[3]);
+      s = nv * fmaf(zz, fq, cr);
+    }
+    cs[c] = s;
+    ci[c] = s > -INFINITY ? v : -1;  // (NaN and -inf are no results, as in the full scan)
+  }
+  __syncthreads();
+  if (tid >= 64) return;
+  // each lane's best of its stride; a round re-reads only the winner's stride
+  float bs = -INFINITY;
+  int bi = INT_MAX, bp = -1;
+  auto scan = [&]() {
+    bs = -INFINITY;
+    bi = INT_MAX;
+    bp = -1;
+    for (int i = tid; i < n; i += 64) {
+      const float s = cs[i];
+      const int id = ci[i];
+      if (id >= 0 && (s > bs || (s == bs && id < bi))) {
+        bs = s;
+        bi = id;
+        bp = i;
+      }
+    }
+  };
+  scan();
+  for (int r = 0; r < k; ++r) {
+    float ms = bs;
+    int mi = bi, mp = bp;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      const float os = __shfl_xor(ms, o, 64);
+      const int oi = __shfl_xor(mi, o, 64), op = __shfl_xor(mp, o, 64);
+      if (op >= 0 && (mp < 0 || os > ms || (os == ms && oi < mi))) {
+        ms = os;
+        mi = oi;
+        mp = op;
+      }
+    }
+    if (tid == 0) {
+      out_s[int64_t(q) * k + r] = mp < 0 ? -INFINITY : ms;
+      out_i[int64_t(q) * k + r] = mp < 0 ? INT_MAX : mi;
+    }
+    if (mp >= 0 && mp == bp) {
+      ci[bp] = -1;
+      scan();
+    }
+  }
+}
+
 }  // namespace
 
 // ------------------------------------------------------------ MIPS search (ABI)
@@ -375,7 +1011,9 @@ __global__ __launch_bounds__(256) void mips_pad(const void* __restrict__ q, int 
 namespace {
 
 struct MipsLayout {
-  int64_t aq, rowc, cs, ci, gth, pad, total;
+  int64_t aq, rowc, cs, ci, gth, pad;
+  int64_t qw, af, ciu, cil, cnt, thr, mx, cand;  // the filter's
+  int64_t total;
 };
 
 // Vector chunks per query tile: enough (query tile, chunk) items for several
@@ -391,7 +1029,81 @@ int mips_splits(int32_t M, int64_t N, int mbits) {
   return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>({want, maxs, 256})));
 }
 
-MipsLayout mips_layout(int32_t M, int d, int mbits, int k, int nsplit) {
+// How a batch of M queries runs: on the full scan, or through the filter with
+// 16 qt queries per wave, wq query tiles and 4 / wq streams per workgroup, pb
+// workgroups (P = 4 pb / wq streams) along the database.
+struct MipsPlan {
+  bool filt;
+  int qt, wq, pb, P, ntile, cap, step;
+};
+
+// Listed vectors a query may have (about 25 k on N(0, 1) data), and the queries
+// per batch that this allows (64 MiB of lists).
+int filt_cap(int k) { return std::max(1024, 64 * k); }
+int filt_batch(int k) { return 16384 * 1024 / filt_cap(k); }
+
+// The filter serves every k <= 64 (its bound comes from 1024 maxima at most):
+// a scan's lists fill at ~0.7 ms per call whatever the size (top-10 of 10^4
+// vectors for 64 queries 753 us, filtered 78; for one query 116 and 49; of 10^6
+// for 10^4 queries 13.1 ms and 3.0), so no smaller search is better off there
+// (N = 2048, one query: 113 and 49 us; k = 1, d = 96: 63 and 38).
+MipsPlan mips_plan(int32_t M, int64_t N, int k) {
+  MipsPlan pl{};
+  pl.filt = k <= kFiltKMax && N >= kFiltMinN;
+  if (!pl.filt) return pl;
+  pl.qt = M <= 16 ? 1 : M <= 64 ? 2 : M <= 1024 ? 4 : kFiltQT;
+  pl.ntile = (M + 16 * pl.qt - 1) / (16 * pl.qt);
+  pl.wq = pl.ntile >= 4 ? 4 : pl.ntile >= 2 ? 2 : 1;
+  pl.cap = filt_cap(k);
+  const int ws = 4 / pl.wq, tg = (pl.ntile + pl.wq - 1) / pl.wq;
+  const int64_t slots = 2 * int64_t(qkv_num_cus());
+  pl.step = N >= kFiltStepN ? kFiltStep : 1;
+  const int64_t ng1 = (N + 16 * pl.step - 1) / (16 * pl.step);  // sampled groups
+  // streams: whole rounds of the chip as nearly as a multiple of 8 allows, at
+  // least 4 k stream maxima, at least one sampled group each
+  const int lo = std::max(8, (k + 4 * ws - 1) / (4 * ws) + 7 & ~7);
+  const int hi = static_cast<int>(std::max<int64_t>(lo, std::min<int64_t>(ng1 / ws, 512)));
+  double best = 0.0;
+  pl.pb = lo;
+  for (int pb = lo; pb <= hi; pb += 8) {
+    const int64_t wg = int64_t(tg) * pb, rounds = (wg + slots - 1) / slots;
+    const double eff = double(wg) / double(rounds * slots) - 0.01 * double(rounds);
+    if (eff > best) {
+      best = eff;
+      pl.pb = pb;
+    }
+  }
+  pl.P = pl.pb * ws;
+  return pl;
+}
+
+// Integer levels of a symmetric codebook: the largest level mapped to 8 .. 100,
+// the others rounded, whichever fits best; false where the QJL weights would
+// need a byte value past 64 (the full scan then runs).
+bool filt_table(const float* kc, int mbits, float qjl_scale, FiltTab* ft) {
+  const int n = 1 << mbits;
+  const float cmax = kc[n - 1];
+  bool found = false;
+  for (int lm = 8; lm <= 100; ++lm) {
+    const float a = cmax / lm;
+    if (!(a > 0.f)) return false;
+    int vlog = 0;
+    while (vlog < 7 && a * (1 << vlog) < 2.f * fabsf(qjl_scale)) ++vlog;
+    if (vlog > 6) continue;
+    uint32_t tab[2] = {0, 0};
+    float delta = 0.f;
+    for (int c = 0; c < n; ++c) {
+      const float l = rintf(kc[c] / a);
+      delta = std::max(delta, fabsf(kc[c] - a * l));
+      tab[c >> 2] |= (static_cast<uint32_t>(static_cast<int>(l)) & 0xffu) << (8 * (c & 3));
+    }
+    if (!found || delta < ft->delta) *ft = FiltTab{tab[0], tab[1], a, delta, lm, vlog};
+    found = true;
+  }
+  return found;
+}
+
+MipsLayout mips_layout(int32_t M, int d, int mbits, int k, int nsplit, const MipsPlan& pl) {
   const int ns = n_odd_subsets(mbits);
   const int64_t nu = 2 * (ns + 1);
   const int64_t chunks = (M + kRowsM - 1) / kRowsM;
@@ -405,6 +1117,17 @@ MipsLayout mips_layout(int32_t M, int d, int mbits, int k, int nsplit) {
   w.gth = off;  off += up(int64_t(M) * 4);
   w.pad = off;  // d < 128: padded queries, Pi and S (fp32)
   if (d < 128) off += up((int64_t(M) * 128 + 128 * 128 + 128) * 4);
+  if (pl.filt) {
+    const int64_t mq = int64_t(pl.ntile) * pl.qt * 16;
+    w.qw = off;   off += up(int64_t(M) * 256 * 4);
+    w.af = off;   off += up(mq / 16 * nu * 64 * 16);
+    w.ciu = off;  off += up(mq * 4);
+    w.cil = off;  off += up(mq * 4);
+    w.cnt = off;  off += up(mq * 4);
+    w.thr = off;  off += up(mq * 4);
+    w.mx = off;   off += up(mq * 16 * pl.P * 4);
+    w.cand = off; off += up(mq * pl.cap * 4);
+  }
   w.total = off;
   return w;
 }
@@ -416,11 +1139,189 @@ int64_t mips_scan_smem(int d, int mbits, int k) {
 
 }  // namespace
 
+namespace {
+
+struct MipsArgs {
+  const void* q;
+  int q_dtype, M, d, mbits;
+  const float* pi;
+  const float* signs;
+  float qjl_scale;
+  const uint8_t* kst;
+  const float* norms;
+  int64_t N;
+  int k;
+  float* out_s;
+  int64_t* out_i;
+};
+
+template <int MB, int PDW>
+int launch_scan(const MipsArgs& a, void* ws, const MipsLayout& L, int nsplit, const int* over,
+                int cap, hipStream_t s) {
+  const int chunks = (a.M + kRowsM - 1) / kRowsM;
+  constexpr int qc = MipsCfg<MB, PDW>::QC;
+  const int64_t vlen = ((a.N + nsplit - 1) / nsplit + kMipsStep - 1) / kMipsStep * kMipsStep;
+  const int64_t qtiles = (chunks + 4 * qc - 1) / (4 * qc);
+  const int64_t n_items = qtiles * nsplit;
+  const int64_t smem = mips_scan_smem(a.d, a.mbits, a.k);
+  int per_cu = 0;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, mips_scan<MB, PDW>, 256,
+                                                   static_cast<size_t>(smem)) != hipSuccess)
+    per_cu = 0;
+  per_cu = std::max(per_cu, 1);
+  const dim3 grid(
+      static_cast<unsigned>(std::min<int64_t>(n_items, int64_t(per_cu) * qkv_num_cus())));
+  if (smem > 65536)
+    QKV_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&mips_scan<MB, PDW>),
+                                hipFuncAttributeMaxDynamicSharedMemorySize,
+                                static_cast<int>(smem)));
+  hipLaunchKernelGGL((mips_scan<MB, PDW>), grid, dim3(256), static_cast<uint32_t>(smem), s,
+                     at<qkv_v4i>(ws, L.aq), at<float>(ws, L.rowc), a.M, a.kst, a.norms, a.N,
+                     nsplit, vlen, n_items, a.k, at<float>(ws, L.cs), at<int>(ws, L.ci),
+                     at<uint32_t>(ws, L.gth), over, cap);
+  QKV_LAUNCHED();
+  const int64_t msmem = int64_t(nsplit) * a.k * 8;
+  if (msmem > 65536)
+    QKV_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&mips_merge),
+                                hipFuncAttributeMaxDynamicSharedMemorySize,
+                                static_cast<int>(std::min<int64_t>(msmem, 160 * 1024))));
+  QKV_REQUIRE(msmem <= 160 * 1024, "too many candidates per query");
+  hipLaunchKernelGGL(mips_merge, dim3(a.M), dim3(64), static_cast<uint32_t>(msmem), s,
+                     at<float>(ws, L.cs), at<int>(ws, L.ci), nsplit, a.k, a.out_s, a.out_i, over,
+                     cap);
+  QKV_LAUNCHED();
+  return QKV_OK;
+}
+
+template <int MB, int PDW, int QT>
+int launch_passes(const MipsArgs& a, void* ws, const MipsLayout& L, const MipsPlan& pl,
+                  const FiltTab& ft, hipStream_t s) {
+  const int tg = (pl.ntile + pl.wq - 1) / pl.wq;
+  const dim3 grid(static_cast<unsigned>(tg * pl.pb));
+  const int64_t ng = (a.N + 15) / 16, ng1 = (ng + pl.step - 1) / pl.step;
+  int* cnt = at<int>(ws, L.cnt);
+  float* thr = at<float>(ws, L.thr);
+  float* mx = at<float>(ws, L.mx);
+  hipLaunchKernelGGL((mips_pass<MB, PDW, QT, false>), grid, dim3(256), 0, s,
+                     at<qkv_v4i>(ws, L.af), at<int>(ws, L.cil), thr, a.kst, a.norms, a.N,
+                     pl.ntile, pl.wq, pl.pb, ng1, pl.step, ft, mx, cnt, at<int>(ws, L.cand),
+                     pl.cap);
+  QKV_LAUNCHED();
+  const unsigned mq = static_cast<unsigned>(pl.ntile * QT * 16);
+  if (a.k <= 16)
+    hipLaunchKernelGGL(mips_bound<1>, dim3(mq), dim3(256), 0, s, mx, 16 * pl.P, a.k, a.M, thr, cnt,
+                       pl.cap);
+  else
+    hipLaunchKernelGGL(mips_bound<4>, dim3(mq), dim3(256), 0, s, mx, 16 * pl.P, a.k, a.M, thr,
+                       cnt, pl.cap);
+  QKV_LAUNCHED();
+  hipLaunchKernelGGL((mips_pass<MB, PDW, QT, true>), grid, dim3(256), 0, s,
+                     at<qkv_v4i>(ws, L.af), at<int>(ws, L.ciu), thr, a.kst, a.norms, a.N,
+                     pl.ntile, pl.wq, pl.pb, ng, 1, ft, mx, cnt, at<int>(ws, L.cand), pl.cap);
+  QKV_LAUNCHED();
+  return QKV_OK;
+}
+
+template <int MB, int PDW>
+int launch_filter(const MipsArgs& a, void* ws, const MipsLayout& L, const MipsPlan& pl,
+                  const FiltTab& ft, hipStream_t s) {
+  int* cnt = at<int>(ws, L.cnt);
+  hipLaunchKernelGGL((mips_fprep<PDW>), dim3(static_cast<unsigned>(pl.ntile * pl.qt)),
+                     dim3(256), 0, s, at<float>(ws, L.qw), at<float>(ws, L.rowc), a.M, ft,
+                     at<uint32_t>(ws, L.af), at<int>(ws, L.ciu), at<int>(ws, L.cil), cnt, pl.cap);
+  QKV_LAUNCHED();
+  int st;
+  switch (pl.qt) {
+    case 1: st = launch_passes<MB, PDW, 1>(a, ws, L, pl, ft, s); break;
+    case 2: st = launch_passes<MB, PDW, 2>(a, ws, L, pl, ft, s); break;
+    case 4: st = launch_passes<MB, PDW, 4>(a, ws, L, pl, ft, s); break;
+    default: st = launch_passes<MB, PDW, kFiltQT>(a, ws, L, pl, ft, s); break;
+  }
+  if (st != QKV_OK) return st;
+  hipLaunchKernelGGL((mips_pick<MB, PDW>), dim3(a.M), dim3(256),
+                     static_cast<uint32_t>(pl.cap * 8), s, at<qkv_v4i>(ws, L.aq),
+                     at<float>(ws, L.rowc), a.kst, a.norms, a.k, cnt, at<int>(ws, L.cand), pl.cap,
+                     a.out_s, a.out_i);
+  QKV_LAUNCHED();
+  return QKV_OK;
+}
+
+int mips_batch(const MipsArgs& a, void* ws, const Tables& tb, hipStream_t s) {
+  MipsPlan pl = mips_plan(a.M, a.N, a.k);
+  const int nsplit = mips_splits(a.M, a.N, a.mbits);
+  const MipsLayout L = mips_layout(a.M, a.d, a.mbits, a.k, nsplit, pl);
+  FiltTab ft{};
+  if (pl.filt) pl.filt = filt_table(tb.kc, a.mbits, a.qjl_scale, &ft);
+  const int chunks = (a.M + kRowsM - 1) / kRowsM;
+  hipLaunchKernelGGL(mips_init, dim3((a.M + 255) / 256), dim3(256), 0, s,
+                     at<uint32_t>(ws, L.gth), a.M);
+  QLayers ql{};
+  ql.q[0] = a.q;
+  ql.pi[0] = a.pi;
+  ql.signs[0] = a.signs;
+  int qdt = a.q_dtype;
+  if (a.d < 128) {
+    float* qp = at<float>(ws, L.pad);
+    float* pip = qp + int64_t(a.M) * 128;
+    float* sp = pip + 128 * 128;
+    const int64_t n = int64_t(a.M) * 128 + 128 * 128 + 128;
+    hipLaunchKernelGGL(mips_pad, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, s,
+                       a.q, a.q_dtype, a.M, a.d, a.pi, a.signs, qp, pip, sp);
+    QKV_LAUNCHED();
+    ql.q[0] = qp;
+    qdt = QKV_F32;
+    ql.pi[0] = pip;
+    ql.signs[0] = sp;
+  }
+  // query operands: the decode prepare kernel with one "kv head" of M rows
+  float* qw = pl.filt ? at<float>(ws, L.qw) : nullptr;
+#define QKV_PREP(NPLV)                                                                           \
+  hipLaunchKernelGGL((prepare_mfma<128, NPLV, false>), dim3(chunks), dim3(256),                  \
+                     (prep_lds<128, NPLV, false>()), s, ql, 1, qdt, a.qjl_scale, a.M, 1, 1, a.M, \
+                     chunks, tb, at<qkv_v4i>(ws, L.aq), at<float>(ws, L.rowc), qw)
+  if (a.mbits == 1) QKV_PREP(2);
+  else if (a.mbits == 2) QKV_PREP(3);
+  else QKV_PREP(5);
+#undef QKV_PREP
+  QKV_LAUNCHED();
+  switch (a.mbits * 10 + a.d / 32) {
+#define QKV_MIPS(MBV, PDWV)                                                                \
+  case MBV * 10 + PDWV:                                                                    \
+    if (pl.filt) {                                                                         \
+      const int st = launch_filter<MBV, PDWV>(a, ws, L, pl, ft, s);                        \
+      if (st != QKV_OK) return st;                                                         \
+    }                                                                                      \
+    return launch_scan<MBV, PDWV>(a, ws, L, nsplit, pl.filt ? at<int>(ws, L.cnt) : nullptr, \
+                                  pl.cap, s);
+    QKV_MIPS(1, 2) QKV_MIPS(1, 3) QKV_MIPS(1, 4)
+    QKV_MIPS(2, 2) QKV_MIPS(2, 3) QKV_MIPS(2, 4)
+    QKV_MIPS(3, 2) QKV_MIPS(3, 3) QKV_MIPS(3, 4)
+#undef QKV_MIPS
+  }
+  return QKV_E_UNSUPPORTED;
+}
+
+// Workspace of M queries: the largest batch's (batches of filt_batch where the
+// filter runs; its plan depends on the batch's size).
+int64_t mips_ws_bytes(int32_t M, int32_t d, int32_t mbits, int32_t k, int64_t N, int32_t* batch) {
+  auto bytes = [&](int32_t m) {
+    return mips_layout(m, d, mbits, k, mips_splits(m, N, mbits), mips_plan(m, N, k)).total;
+  };
+  *batch = M;
+  const int32_t most = filt_batch(k);
+  if (M <= most || !mips_plan(M, N, k).filt) return bytes(M);
+  *batch = most;
+  const int32_t rest = M % most;
+  return std::max(bytes(most), rest > 0 ? bytes(rest) : 0);
+}
+
+}  // namespace
+
 extern "C" int64_t qkv_mips_workspace_bytes(int32_t M, int32_t d, int32_t mbits, int32_t k,
                                             int64_t N) {
   if (M <= 0 || !qkv_d_ok(d) || mbits < 1 || mbits > 3 || k <= 0 || N <= 0) return -1;
-  const int kk = static_cast<int>(std::min<int64_t>(k, N));
-  return mips_layout(M, d, mbits, kk, mips_splits(M, N, mbits)).total;
+  int32_t batch = 0;
+  return mips_ws_bytes(M, d, mbits, static_cast<int>(std::min<int64_t>(k, N)), N, &batch);
 }
 
 extern "C" int qkv_mips_search(const void* queries, int32_t q_dtype, int32_t M, int32_t d,
@@ -455,100 +1356,17 @@ extern "C" int qkv_mips_search(const void* queries, int32_t q_dtype, int32_t M, 
     return QKV_E_UNSUPPORTED;
   }
   tb.mfma_ok = 1;
-  const int nsplit = mips_splits(M, N, mbits);
-  const MipsLayout L = mips_layout(M, d, mbits, k, nsplit);
-  QKV_REQUIRE(ws_bytes >= L.total, "workspace too small: %lld < %lld", (long long)ws_bytes,
-              (long long)L.total);
-  auto s = static_cast<hipStream_t>(stream);
-  const int chunks = (M + kRowsM - 1) / kRowsM;
-  qkv_v4i* aq = at<qkv_v4i>(workspace, L.aq);
-  float* rowc = at<float>(workspace, L.rowc);
-  float* cs = at<float>(workspace, L.cs);
-  int* ci = at<int>(workspace, L.ci);
-  uint32_t* gth = at<uint32_t>(workspace, L.gth);
-  hipLaunchKernelGGL(mips_init, dim3((M + 255) / 256), dim3(256), 0, s, gth, M);
-  const void* qsrc = queries;
-  int qdt = q_dtype;
-  const float* pisrc = pi;
-  const float* ssrc = signs;
-  if (d < 128) {
-    float* qp = at<float>(workspace, L.pad);
-    float* pip = qp + int64_t(M) * 128;
-    float* sp = pip + 128 * 128;
-    const int64_t n = int64_t(M) * 128 + 128 * 128 + 128;
-    hipLaunchKernelGGL(mips_pad, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, s,
-                       queries, q_dtype, M, d, pi, signs, qp, pip, sp);
-    QKV_LAUNCHED();
-    qsrc = qp;
-    qdt = QKV_F32;
-    pisrc = pip;
-    ssrc = sp;
+  int32_t batch = 0;
+  const int64_t need = mips_ws_bytes(M, d, mbits, k, N, &batch);
+  QKV_REQUIRE(ws_bytes >= need, "workspace too small: %lld < %lld", (long long)ws_bytes,
+              (long long)need);
+  const int esize = q_dtype == QKV_F32 ? 4 : 2;
+  for (int32_t m0 = 0; m0 < M; m0 += batch) {
+    MipsArgs a{static_cast<const char*>(queries) + int64_t(m0) * d * esize,
+               q_dtype, std::min(batch, M - m0), d, mbits, pi, signs, qjl_scale, kstore, norms, N,
+               k, out_scores + int64_t(m0) * k, out_indices + int64_t(m0) * k};
+    const int st = mips_batch(a, workspace, tb, static_cast<hipStream_t>(stream));
+    if (st != QKV_OK) return st;
   }
-  // query operands: the decode prepare kernel with one "kv head" of M rows
-  QLayers ql{};
-  ql.q[0] = qsrc;
-  ql.pi[0] = pisrc;
-  ql.signs[0] = ssrc;
-#define QKV_PREP(NPLV)                                                                        \
-  hipLaunchKernelGGL((prepare_mfma<128, NPLV, false>), dim3(chunks), dim3(256),                     \
-                     (prep_lds<128, NPLV, false>()), s, ql, 1, qdt,                                \
-                     qjl_scale, M, 1, 1, M, chunks, tb, aq, rowc, nullptr)
-  if (mbits == 1) QKV_PREP(2);
-  else if (mbits == 2) QKV_PREP(3);
-  else QKV_PREP(5);
-#undef QKV_PREP
-  QKV_LAUNCHED();
-  const int qc = mbits <= 2 ? 4 : 2;
-  const int64_t vlen = ((N + nsplit - 1) / nsplit + kMipsStep - 1) / kMipsStep * kMipsStep;
-  const int64_t qtiles = (chunks + 4 * qc - 1) / (4 * qc);
-  const int64_t n_items = qtiles * nsplit;
-  const int64_t smem = mips_scan_smem(d, mbits, k);
-  int per_cu = 0;
-  switch (mbits * 10 + d / 32) {
-#define QKV_OCC(MBV, PDWV, CASEV)                                                         \
-  case CASEV:                                                                             \
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, mips_scan<MBV, PDWV>, 256,  \
-                                                     static_cast<size_t>(smem)) != hipSuccess) \
-      per_cu = 0;                                                                         \
-    break;
-    QKV_OCC(1, 2, 12) QKV_OCC(1, 3, 13) QKV_OCC(1, 4, 14)
-    QKV_OCC(2, 2, 22) QKV_OCC(2, 3, 23) QKV_OCC(2, 4, 24)
-    QKV_OCC(3, 2, 32) QKV_OCC(3, 3, 33) QKV_OCC(3, 4, 34)
-#undef QKV_OCC
-  }
-  per_cu = std::max(per_cu, 1);
-  const dim3 grid(static_cast<unsigned>(
-      std::min<int64_t>(n_items, int64_t(per_cu) * qkv_num_cus())));
-#define QKV_SCAN(MBV, PDWV)                                                                       \
-  do {                                                                                            \
-    if (smem > 65536)                                                                             \
-      QKV_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&mips_scan<MBV, PDWV>),          \
-                                  hipFuncAttributeMaxDynamicSharedMemorySize,                     \
-                                  static_cast<int>(smem)));                                       \
-    hipLaunchKernelGGL((mips_scan<MBV, PDWV>), grid, dim3(256), static_cast<uint32_t>(smem), s,  \
-                       aq, rowc, M, kstore, norms, N, nsplit, vlen, n_items, k, cs, ci, gth);     \
-  } while (0)
-  switch (mbits * 10 + d / 32) {
-    case 12: QKV_SCAN(1, 2); break;
-    case 13: QKV_SCAN(1, 3); break;
-    case 14: QKV_SCAN(1, 4); break;
-    case 22: QKV_SCAN(2, 2); break;
-    case 23: QKV_SCAN(2, 3); break;
-    case 24: QKV_SCAN(2, 4); break;
-    case 32: QKV_SCAN(3, 2); break;
-    case 33: QKV_SCAN(3, 3); break;
-    case 34: QKV_SCAN(3, 4); break;
-  }
-#undef QKV_SCAN
-  QKV_LAUNCHED();
-  const int64_t msmem = int64_t(nsplit) * k * 8;
-  if (msmem > 65536)
-    QKV_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&mips_merge),
-                                hipFuncAttributeMaxDynamicSharedMemorySize,
-                                static_cast<int>(std::min<int64_t>(msmem, 160 * 1024))));
-  QKV_REQUIRE(msmem <= 160 * 1024, "too many candidates per query");
-  hipLaunchKernelGGL(mips_merge, dim3(M), dim3(64), static_cast<uint32_t>(msmem), s, cs, ci,
-                     nsplit, k, out_scores, out_indices);
-  QKV_LAUNCHED();
   return QKV_OK;
 }
