@@ -40,6 +40,7 @@
 #include <mutex>
 
 #include "qkv_attn_prep.h"
+#include "qkv_prefill.h"
 
 
 namespace {
@@ -2204,8 +2205,13 @@ int launch_fused(const QLayers& ql, const KVLayers& kv, const OutLayers& ol, int
 
 // ------------------------------------------------------------ C ABI
 
-extern "C" int32_t qkv_attention_splits(int32_t B, int32_t Hq, int32_t Hkv, int32_t Q,
-                                        int32_t d, int64_t T) {
+int combine_layers(const OutLayers& ol, int nl, int32_t B, int32_t Hq, int32_t Hkv, int32_t Q,
+                   int32_t d, int32_t out_dtype, void* workspace, int64_t ws_bytes,
+                   int32_t n_splits, hipStream_t s);
+
+// Splits of the decode kernels (4 or 8 query rows per workgroup).
+static int32_t decode_splits(int32_t B, int32_t Hq, int32_t Hkv, int32_t Q, int32_t d,
+                             int64_t T) {
   if (B <= 0 || Hkv <= 0 || Hq <= 0 || Q <= 0 || T <= 0) return 1;
   const int R = (Hq / Hkv) * Q;
   if (d == 128 || d == 96)
@@ -2219,6 +2225,77 @@ extern "C" int32_t qkv_attention_splits(int32_t B, int32_t Hq, int32_t Hkv, int3
   int64_t sp = std::min<int64_t>((2 * ncu + groups - 1) / groups, (T + kChunkS - 1) / kChunkS);
   sp = std::max<int64_t>(sp, (T + kSplitMax - 1) / kSplitMax);
   return static_cast<int32_t>(std::max<int64_t>(1, std::min<int64_t>(sp, 1024)));
+}
+
+// Whether the prefill kernel is the faster one for R query rows in each of bh
+// (sequence, kv head) groups over T keys: both kernels' times in us as measured
+// (rounds of the chip's workgroups times their steps; fixed part; the merge of
+// splits).  E.g. d = 128, 8 groups: 48 rows over 256 keys 19 against 28 us, over
+// 8192 keys 51 against 37; 256 rows over 2048 keys 42 against 39; 8192 rows over
+// 2048 keys 1052 against 144.
+static bool prefill_pays(int32_t B, int32_t Hq, int32_t Hkv, int32_t Q, int32_t d, int64_t T) {
+  const int R = (Hq / Hkv) * Q;
+  if (R < kPrefillMinRows || !qkv_d_ok(d)) return false;
+  const int64_t bh = int64_t(B) * Hkv, ncu = qkv_num_cus();
+  auto rounds = [&](int64_t wgs) { return static_cast<double>((wgs + ncu - 1) / ncu); };
+  const int ds = decode_splits(B, Hq, Hkv, Q, d, T);
+  double dec;
+  if (d == 64) {  // decode_small: 8 rows per workgroup, three workgroups per CU
+    dec = 12.0 + 2.7e-5 * double(bh * ((R + 7) / 8)) * double(T);
+  } else {        // decode_fused: 4 rows, 512-token chunks of 2.31 us
+    dec = rounds(bh * ((R + kRowsM - 1) / kRowsM) * ds) *
+          (11.0 + 2.31 / 512.0 * double(T) / ds);
+  }
+  dec += ds > 1 ? 5.0 : 0.0;
+  const int ps = qkv_prefill_splits(bh, R, d, T);
+  const double step = d == 128 ? 4.4 : d == 96 ? 3.2 : 2.0;  // per 64 tokens
+  const double r = rounds(bh * ((R + 127) / 128) * ps);
+  const double pre = 2.0 + r * (8.0 + step * double((T + 64 * ps - 1) / (64 * ps))) +
+                     (ps > 1 ? 5.0 + 2.5e-7 * double(bh) * R * d * 8 * ps : 0.0);
+  return pre < dec;
+}
+
+extern "C" int32_t qkv_attention_splits(int32_t B, int32_t Hq, int32_t Hkv, int32_t Q,
+                                        int32_t d, int64_t T) {
+  if (B <= 0 || Hkv <= 0 || Hq <= 0 || Q <= 0 || T <= 0) return 1;
+  if (prefill_pays(B, Hq, Hkv, Q, d, T))
+    return qkv_prefill_splits(int64_t(B) * Hkv, (Hq / Hkv) * Q, d, T);
+  return decode_splits(B, Hq, Hkv, Q, d, T);
+}
+
+// The prefill kernel's calls: one layer, codebooks it takes.  Its splits follow
+// its own rule (128 rows per workgroup), so a call it would have had but that
+// stays on the decode kernels has them cut to theirs.
+static bool use_prefill(int32_t B, int32_t Hq, int32_t Hkv, int32_t Q, int32_t d, int64_t T,
+                        int32_t kbits, int32_t vbits, const float* kcent, const float* vcent,
+                        float qjl_scale, int64_t t_stride) {
+  return prefill_pays(B, Hq, Hkv, Q, d, T) && t_stride % 64 == 0 &&
+         qkv_prefill_ok(d, kbits, vbits, kcent, vcent, qjl_scale);
+}
+static int clamp_splits(int32_t B, int32_t Hq, int32_t Hkv, int32_t Q, int32_t d, int64_t T,
+                        int n_splits) {
+  if (!prefill_pays(B, Hq, Hkv, Q, d, T)) return n_splits;
+  return std::min<int>(n_splits, decode_splits(B, Hq, Hkv, Q, d, T));
+}
+static int run_prefill(const void* q, int32_t q_dtype, const KVLayers& kv, int64_t t_stride,
+                       int64_t T, int32_t B, int32_t Hq, int32_t Hkv, int32_t Q, int32_t d,
+                       int32_t kbits, int32_t vbits, const float* pi, const float* kcent,
+                       const float* vcent, const float* signs, float qjl_scale, float scale,
+                       int32_t causal, void* out, int32_t out_dtype, void* workspace,
+                       int64_t ws_bytes, int32_t n_splits, hipStream_t s) {
+  QKV_REQUIRE(qkv_aligned(pi, 16) && qkv_aligned(kv.kst[0], 4) && qkv_aligned(kv.vst[0], 4),
+              "pi must be 16-byte and the store 4-byte aligned");
+  const WsLayout L = ws_layout(B, Hkv, (Hq / Hkv) * Q, d, n_splits);
+  QkvPrefillArgs a{q,    q_dtype, kv,    t_stride,  T,     B,      Hq,  Hkv,       Q,
+                   d,    kbits,   vbits, pi,        kcent, vcent,  signs, qjl_scale, scale,
+                   causal, out,   out_dtype, n_splits, at<float>(workspace, L.po),
+                   at<float>(workspace, L.pml)};
+  const int st = qkv_prefill(a, s);
+  if (st != QKV_OK || n_splits == 1) return st;
+  OutLayers ol{};
+  ol.pi[0] = pi;
+  ol.out[0] = out;
+  return combine_layers(ol, 1, B, Hq, Hkv, Q, d, out_dtype, workspace, ws_bytes, n_splits, s);
 }
 
 extern "C" int64_t qkv_attention_workspace_bytes(int32_t B, int32_t Hq, int32_t Hkv, int32_t Q,
@@ -2533,6 +2610,12 @@ int decode_attention_impl(const void* q, int32_t q_dtype, const uint8_t* kstore,
   kv.khi = kr.khi;
   kv.cbase = kr.cbase;
   auto s = static_cast<hipStream_t>(stream);
+  if (use_prefill(B, Hq, Hkv, Q, d, T, kbits, vbits, kcent_host, vcent_host, qjl_scale,
+                  t_stride))
+    return run_prefill(q, q_dtype, kv, t_stride, T, B, Hq, Hkv, Q, d, kbits, vbits, pi,
+                       kcent_host, vcent_host, signs, qjl_scale, scale, causal, out, out_dtype,
+                       workspace, ws_bytes, n_splits, s);
+  n_splits = clamp_splits(B, Hq, Hkv, Q, d, T, n_splits);
   const Tables tb = make_tables(kcent_host, kbits, vcent_host, vbits);
   if (d == 64 && tb.mfma_ok && t_stride % 64 == 0 && !kr.klo && !kr.khi && kr.cbase == 0) {
     // decode_small: one launch (plus combine_kernel with several splits)
@@ -2668,8 +2751,12 @@ extern "C" int qkv_decode_attention_noalloc(const void* q, int32_t q_dtype,
                                             int32_t n_splits, void* stream) {
   QKV_REQUIRE(B > 0 && Hq > 0 && Hkv > 0 && Q > 0 && Hq % Hkv == 0, "invalid shape");
   QKV_REQUIRE(n_splits >= 1 && n_splits <= 1024, "n_splits %d out of range", n_splits);
-  const int64_t need = qkv_attention_workspace_bytes(B, Hq, Hkv, Q, d, n_splits);
+  int64_t need = qkv_attention_workspace_bytes(B, Hq, Hkv, Q, d, n_splits);
   QKV_REQUIRE(need > 0, "invalid shape");
+  // the prefill kernel's splits are a matter of speed only: as many as fit
+  while (need > int64_t(QKV_NOALLOC_SCRATCH_BYTES) && n_splits > 1 &&
+         prefill_pays(B, Hq, Hkv, Q, d, T))
+    need = qkv_attention_workspace_bytes(B, Hq, Hkv, Q, d, --n_splits);
   QKV_REQUIRE(need <= int64_t(QKV_NOALLOC_SCRATCH_BYTES),
               "qkv_decode_attention_noalloc: this call needs %lld workspace bytes, more than "
               "the %lld-byte scratch array (use qkv_decode_attention with a workspace)",
@@ -2724,6 +2811,12 @@ extern "C" int qkv_paged_decode_attention(
   kv.pmax = pages_per_seq;
   kv.plg = plg;
   kv.npages = num_pages;
+  if (use_prefill(B, Hq, Hkv, Q, d, T, kbits, vbits, kcent_host, vcent_host, qjl_scale,
+                  t_stride))
+    return run_prefill(q, q_dtype, kv, t_stride, T, B, Hq, Hkv, Q, d, kbits, vbits, pi,
+                       kcent_host, vcent_host, signs, qjl_scale, scale, causal, out, out_dtype,
+                       workspace, ws_bytes, n_splits, static_cast<hipStream_t>(stream));
+  n_splits = clamp_splits(B, Hq, Hkv, Q, d, T, n_splits);
   {  // the kernels of the contiguous single call: decode_small at d = 64 with
      // key MSE bits <= 2, decode_fused otherwise
     QLayers ql{};
@@ -2793,6 +2886,7 @@ static int decode_layers(int32_t n_layers, const void* const* q, int32_t q_dtype
                   "bits <= 3, capacity a multiple of 64)");
     return QKV_E_UNSUPPORTED;
   }
+  n_splits = clamp_splits(B * n_layers, Hq, Hkv, Q, d, T, n_splits);
   QLayers ql{};
   KVLayers kv{};
   OutLayers ol{};
@@ -2908,6 +3002,7 @@ int kmixed_decode_impl(int kind, const void* q, int32_t q_dtype, const uint8_t* 
   }
   QKV_REQUIRE(qkv_aligned(pi_perm, 16) && qkv_aligned(pi_v, 16), "pi must be 16-byte aligned");
   QKV_REQUIRE(qkv_aligned(kstore, 4), "K rows must be 4-byte aligned");
+  n_splits = clamp_splits(B, Hq, Hkv, Q, d, T, n_splits);
   QLayers ql{};
   ql.q[0] = q;
   ql.pi[0] = pi_perm;

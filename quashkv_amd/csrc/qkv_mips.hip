@@ -382,6 +382,9 @@ __global__ __launch_bounds__(64) void mips_merge(const float* __restrict__ cand_
 // registers and streams 16-vector groups from L2 into registers two groups
 // ahead; no barrier, so the waves drift apart and one's VALU overlaps another's
 // MFMAs.
+// (the HIP headers' min of 64-bit integers goes through double)
+__device__ __forceinline__ int64_t imin(int64_t a, int64_t b) { return a < b ? a : b; }
+
 constexpr int kNoI = -(1 << 30);   // no value of I (|I| < 2^22) brings it to 0
 constexpr int kFiltStep = 8;       // groups per sampled group of pass 1, from
 constexpr int64_t kFiltStepN = 8192;     // this many vectors (below, pass 1 takes every group)
@@ -565,9 +568,9 @@ __global__ __launch_bounds__(256, 2) void mips_pass(
   const uint32_t wo = PDW == 2 ? (lg & 1) : PDW == 3 ? min(lg, 2) : lg;
   auto load = [&](int64_t x) {
     Row r;
-    const int64_t v0 = min<int64_t>(x, ng - 1) * gstep * 16;
+    const int64_t v0 = imin(x, ng - 1) * gstep * 16;
     // (the last group may be partial; no branch, which would split the schedule)
-    const uint32_t left = static_cast<uint32_t>(min<int64_t>(N - 1 - v0, 15));
+    const uint32_t left = static_cast<uint32_t>(imin(N - 1 - v0, 15));
     const uint32_t ni = min<uint32_t>(ln, left), lo = (ni * RAWD + wo) * 4;
     const uint8_t* base = kst + v0 * (RAWD * 4);
 #pragma unroll

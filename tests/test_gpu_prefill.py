@@ -1,0 +1,177 @@
+"""Attention of many query rows per kv head (the prefill kernel) against softmax
+attention in 64 bits over the store's own codes: every head dim, key and value
+width, query and output dtype, GQA group, remainders of the 128-row and 32-token
+tiles, causal and full, key ranges, splits, paged stores, large logits.
+
+The shapes have enough (sequence, kv head) groups that the dispatch's cost rule
+sends them to the prefill kernel (smaller calls stay on the decode kernels).
+
+Bar for fp32 outputs: 3e-5 relative (2-norm), the decode kernels' own (their
+large-logit bar is 1e-4, measured 2.2e-5)."""
+
+import math
+
+import pytest
+import torch
+
+import quashkv_amd as quashkv
+from quashkv_amd import _native as N
+from quashkv_amd.kernels import attention_store
+from quashkv_amd.paged import PagedQuashKVEngine
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda"
+
+
+@pytest.fixture(autouse=True, scope="module")
+def _need_gpu():
+    if not torch.cuda.is_available():
+        pytest.skip("needs a HIP device")
+    N.lib()
+
+
+def exact(e, q, causal, lo=None, hi=None, q_end=0, signs=None, logits=False):
+    b0 = e._cache[0]
+    kc = torch.cat([b.mse_indices for b in e._cache], 2).long()
+    vc = torch.cat([b.val_indices for b in e._cache], 2).long()
+    kn = torch.cat([b.key_norms for b in e._cache], 2).double()
+    vn = torch.cat([b.val_norms for b in e._cache], 2).double()
+    qs = torch.cat([b.qjl_signs for b in e._cache], 2).double()
+    assert b0.qjl_signs is not None
+    kq, vq = e.key_quantizer, e.value_quantizer
+    mq = kq.mse_quantizer
+    S = (kq.S if signs is None else signs).double()
+    B, Hq, Q, d = q.shape
+    Hkv, T = kc.shape[1:3]
+    G = Hq // Hkv
+    k = mq.codebook.centroids.double()[kc].repeat_interleave(G, 1)
+    sg = ((2 * qs - 1) * S).repeat_interleave(G, 1)
+    v = (vq.codebook.centroids.double()[vc] * vn[..., None]).repeat_interleave(G, 1)
+    qr = q.double() @ mq.Pi.double().T
+    s = qr @ k.transpose(2, 3) + kq.qjl_scale * (qr.abs() @ sg.transpose(2, 3))
+    s = s * kn.repeat_interleave(G, 1)[:, :, None] / math.sqrt(d)
+    top = float(s.abs().max())
+    t = torch.arange(T, device=q.device)
+    lo = torch.zeros(B, device=q.device) if lo is None else lo
+    hi = torch.full((B,), T, device=q.device) if hi is None else hi
+    end = hi if q_end == 0 else torch.full_like(hi, q_end)
+    dead = (t[None, :] < lo[:, None]) | (t[None, :] >= hi[:, None])
+    dead = dead[:, None, None, :].expand(B, 1, Q, T)
+    if causal:
+        pos = end[:, None] - Q + torch.arange(Q, device=q.device)[None]
+        dead = dead | (t[None, None, :] > pos[:, :, None])[:, None]
+    s = s.masked_fill(dead, -math.inf)
+    p = torch.nan_to_num(torch.softmax(s, -1))   # a row with no keys: zeros
+    out = (p @ v) @ vq.Pi.double()
+    return (out, top) if logits else out
+
+
+def check(out, ref, bar=3e-5):
+    err = float((out.double() - ref).norm() / ref.norm())
+    assert err <= bar, err
+
+
+def filled(B, H, T, d, kb, vb, seed, dtype=torch.bfloat16, cls=quashkv.QuashKVEngine, **kw):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    e = cls(head_dim=d, key_bits=kb, value_bits=vb, seed=11, device=DEV, **kw)
+    k = torch.randn(B, H, T, d, device=DEV, generator=g)
+    k[..., ::32] *= 10.0
+    v = torch.randn(B, H, T, d, device=DEV, generator=g)
+    e.append(k.to(dtype), v.to(dtype))
+    return e, g
+
+
+@pytest.mark.parametrize("d", [64, 96, 128])
+@pytest.mark.parametrize("kb,vb", [(2, 1), (2, 2), (3, 3), (3, 4), (4, 4), (4, 2)])
+@pytest.mark.parametrize("B,G,H,T,Q,causal,dtype", [
+    (8, 4, 8, 160, 33, True, torch.bfloat16),   # 132 rows: a 4-row remainder
+    (20, 7, 5, 95, 41, False, torch.float16),
+    (11, 1, 9, 300, 129, True, torch.float32),
+])
+def test_prefill_matches_64_bits(d, kb, vb, B, G, H, T, Q, causal, dtype):
+    e, g = filled(B, H, T, d, kb, vb, T + Q)
+    q = torch.randn(B, H * G, Q, d, device=DEV, generator=g).to(dtype)
+    ref = exact(e, q, causal)
+    check(e.attention(q, causal=causal), ref)
+    check(e.attention(q, causal=causal, out_dtype=torch.bfloat16).float(), ref, 4e-3)
+    check(e.attention(q, causal=causal, out_dtype=torch.float16).float(), ref, 6e-4)
+
+
+@pytest.mark.parametrize("T,Q,G", [(48, 48, 1), (64, 12, 4), (31, 31, 2), (1024, 16, 8),
+                                   (2048, 300, 1), (1500, 1500, 2)])
+def test_prefill_sizes(T, Q, G):
+    """The smallest calls, whole and odd numbers of tiles, Q = T."""
+    e, g = filled(8, 8, T, 128, 3, 3, T)
+    q = torch.randn(8, 8 * G, Q, 128, device=DEV, generator=g)
+    check(e.attention(q, causal=True), exact(e, q, True))
+
+
+@pytest.mark.parametrize("d,splits", [(128, 2), (128, 7), (96, 3), (64, 64)])
+def test_prefill_splits(d, splits):
+    e, g = filled(8, 8, 700, d, 3, 3, splits)
+    q = torch.randn(8, 32, 60, d, device=DEV, generator=g)
+    kq, vq = e.key_quantizer, e.value_quantizer
+    for causal in (False, True):
+        out = attention_store(q, e._store, 700, kq.mse_quantizer.Pi,
+                              kq.mse_quantizer.codebook.centroids_host,
+                              vq.codebook.centroids_host, kq.S, kq.qjl_scale, causal=causal,
+                              n_splits=splits)
+        check(out, exact(e, q, causal))
+
+
+def test_prefill_ranges_and_positions():
+    e, g = filled(4, 16, 333, 128, 3, 3, 5)
+    q = torch.randn(4, 64, 40, 128, device=DEV, generator=g)
+    lo = torch.tensor([0, 31, 32, 200], device=DEV, dtype=torch.int32)
+    hi = torch.tensor([333, 300, 97, 200], device=DEV, dtype=torch.int32)   # the last: no keys
+    for causal, q_end in ((False, 0), (True, 0), (True, 333), (True, 60)):
+        out = e.attention(q, causal=causal, kv_start=lo, kv_end=hi, q_end=q_end)
+        check(out, exact(e, q, causal, lo, hi, q_end))
+        assert float(out[3].abs().max()) == 0.0
+
+
+@pytest.mark.parametrize("d,kb,page", [(128, 3, 64), (96, 4, 256), (64, 3, 2048)])
+def test_prefill_paged_equals_contiguous(d, kb, page):
+    args = (8, 8, 515, d, kb, 3, 7)
+    a, g = filled(*args)
+    b, _ = filled(*args, cls=PagedQuashKVEngine, page_tokens=page)
+    q = torch.randn(8, 32, 60, d, device=DEV, generator=g)
+    assert torch.equal(a.attention(q, causal=True), b.attention(q, causal=True))
+
+
+@pytest.mark.parametrize("kb,vb", [(2, 2), (3, 3), (4, 4)])
+def test_prefill_large_logits_and_norms(kb, vb):
+    """Key and value norms over eight decades, tiny and huge queries."""
+    g = torch.Generator(device=DEV).manual_seed(9)
+    e = quashkv.QuashKVEngine(head_dim=128, key_bits=kb, value_bits=vb, seed=3, device=DEV)
+    T = 777
+    k = torch.randn(8, 8, T, 128, device=DEV, generator=g)
+    v = torch.randn(8, 8, T, 128, device=DEV, generator=g)
+    k *= torch.exp(1.5 * torch.randn(8, 8, T, 1, device=DEV, generator=g))
+    v *= torch.logspace(-4, 4, T, device=DEV)[torch.randperm(T, device=DEV, generator=g)][:, None]
+    e.append(k, v)
+    q = torch.randn(8, 32, 50, 128, device=DEV, generator=g)
+    q[:, :, 1] *= 1e-6
+    q[:, :, 2, 1:] = 0.0
+    q[:, :, 3] = 0.0
+    ref, top = exact(e, q, True, logits=True)
+    out = e.attention(q, causal=True)
+    err = (out.double() - ref).norm(dim=-1) / ref.norm(dim=-1).clamp(min=1e-30)
+    # a score is good to 4e-6 of itself (the f16 key levels: 1e-6, and 2.5e-5 of the
+    # QJL term, a ninth of it), so a row moves by at most that of the largest logit;
+    # the decode kernels' error here is 3e-2 on average
+    assert float(err.max()) <= 4e-6 * top + 2e-5 and float(err.mean()) <= 2e-5
+
+
+def test_prefill_other_signs():
+    """S that f16 does not hold exactly (and of size 0): the third QJL product."""
+    e, g = filled(8, 8, 200, 128, 3, 3, 5)
+    q = torch.randn(8, 32, 30, 128, device=DEV, generator=g)
+    kq, vq = e.key_quantizer, e.value_quantizer
+    signs = kq.S * (0.5 + torch.rand(128, device=DEV, generator=g))
+    signs[5] = 0.0
+    out = attention_store(q, e._store, 200, kq.mse_quantizer.Pi,
+                          kq.mse_quantizer.codebook.centroids_host, vq.codebook.centroids_host,
+                          signs, kq.qjl_scale, causal=True)
+    check(out, exact(e, q, True, signs=signs))
