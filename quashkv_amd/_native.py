@@ -299,7 +299,7 @@ class HostInts:
 
 def ptr_array(ptrs) -> "ctypes.Array":
     """Device pointers (ints) as a host array of void* (per-layer arguments)."""
-    return (ctypes.c_void_p * max(len(ptrs), 1))(*[ctypes.c_void_p(int(x)) for x in ptrs])
+    return (ctypes.c_void_p * max(len(ptrs), 1))(*ptrs)
 
 
 def packed_row_bytes(d: int, bits: int) -> int:
