@@ -439,8 +439,11 @@ __device__ __forceinline__ void mma_store(const uint4 (&ah)[R][Geo<D>::NK],
     const int q = lane % cpr;
     for (int v = lane / cpr; v < 16 * R; v += rows) {
       const uint4 w = *reinterpret_cast<const uint4*>(ost + v * rsb + 16 * q);
+      // non-temporal (aux 2): rows that fill whole lines and outgrow the caches;
+      // without it the write-backs share the L2 with the codes' reads (524,288 rows
+      // of K and of V, d = 128, fp32: 188 -> 159 us, and 195 -> 148 on another card)
       __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(qkv_u32x4, w), ob,
-                                             (v * D + 32 * p) * obytes + 16 * q, 0, 0);
+                                             (v * D + 32 * p) * obytes + 16 * q, 0, 2);
     }
   }
 }
