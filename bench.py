@@ -796,7 +796,7 @@ def sub_cfg5(args, dev, stream) -> dict:
     for c in range(0, M, 1000):
         ex = torch.topk(qs[c:c + 1000] @ db.T, K, dim=1).indices
         hits += int((ix[c:c + 1000].unsqueeze(2) == ex.unsqueeze(1)).any(dim=2).sum())
-    ops = 2.0 * M * NV * 384 * 4      # int8 MACs of the bit-plane dot products, x2
+    ops = 2.0 * M * NV * 256 * 1.125  # int8 MACs of the filter's two passes, x2
     res = {
         "what": "QuashIndex MIPS: 10^6 x 128 L2-normalised vectors, 3-bit (2-bit MSE + QJL), "
                 "10^4 queries, exhaustive top-10",
