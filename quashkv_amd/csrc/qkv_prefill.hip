@@ -66,6 +66,8 @@ constexpr int kTok = 32;      // tokens per wave and step
 constexpr int kStep = 64;     // tokens per workgroup and step
 constexpr int kThr = 512;
 constexpr int kRowsWg = 128;
+constexpr float kMinNorm = 0x1p-90f;  // |v| as the softmax reference sees it
+constexpr int kMinExp = -123;         // of a row's scale: its inverse stays finite
 constexpr float kHead = 8.f;  // the running maximum may lag by 2^8 before a rescale
 
 // f16 levels of a codebook: bytes of the f16 values of codes 0 .. 7 (16-level
@@ -307,6 +309,7 @@ __global__ __launch_bounds__(kThr, 2) void prefill(PreArgs A, KVLayers kv) {
     amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
     int ex = 0;
     if (amax > 0.f && amax < INFINITY) frexpf(amax, &ex);
+    ex = max(ex, kMinExp);
     const float up = ldexpf(1.f, 3 - ex);  // the row's largest into [4, 8)
     fr = ldexpf(1.f, ex - 3);
     v4u xh[KK], xl[KK];
@@ -447,7 +450,8 @@ __global__ __launch_bounds__(kThr, 2) void prefill(PreArgs A, KVLayers kv) {
         r.v[k] = *reinterpret_cast<const uint32_t*>(vs + (vofs + 4 * D * k));
     }
     r.nm = 0.f;
-    if (wave < 2 && h == 0 && t + perm32(n) < A.T)
+    // (0 outside the key range: its slots may hold anything)
+    if (wave < 2 && h == 0 && t + perm32(n) >= sr.lo && t + perm32(n) < sr.hi)
       r.nm = (wave == 0 ? kv.knorm[0] : kv.vnorm[0])[row + perm32(n)];
     return r;
   };
@@ -483,7 +487,8 @@ __global__ __launch_bounds__(kThr, 2) void prefill(PreArgs A, KVLayers kv) {
     if (wave < 2) {
       if (h == 0) {
         nm[32 * wave + n] = wave == 0 ? r.nm * A.c0 : r.nm;
-        if (wave == 1) nm[64 + n] = __builtin_amdgcn_logf(fabsf(r.nm));  // log2; -inf at 0
+        // log2, from 2^-90 up: a row of zero norms alone keeps finite weights
+        if (wave == 1) nm[64 + n] = __builtin_amdgcn_logf(fmaxf(fabsf(r.nm), kMinNorm));
       }
     }
   };
@@ -690,6 +695,7 @@ __global__ __launch_bounds__(kThr, 2) void prefill(PreArgs A, KVLayers kv) {
     amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
     int ex = 0;
     if (amax > 0.f && amax < INFINITY) frexpf(amax, &ex);
+    ex = max(ex, kMinExp);
     const float up = ldexpf(1.f, 3 - ex);
     *rsc = ldexpf(1.f, ex - 9);  // (Pi is scaled by 64)
 #pragma unroll

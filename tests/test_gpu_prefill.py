@@ -175,3 +175,26 @@ def test_prefill_other_signs():
                           kq.mse_quantizer.codebook.centroids_host, vq.codebook.centroids_host,
                           signs, kq.qjl_scale, causal=True)
     check(out, exact(e, q, True, signs=signs))
+
+
+@pytest.mark.parametrize("d,T", [(64, 200), (128, 333)])
+def test_prefill_extremes(d, T):
+    """Value norms of zero (rows that see no other among them), queries below 1e-38,
+    and slots outside the key range whose norms are not finite."""
+    e, g = filled(8, 8, T, d, 3, 3, 13, dtype=torch.float32)
+    st = e._store
+    st.vnorm.view(8, 8, -1)[:, :, :40] = 0.0
+    q = torch.randn(8, 32, 80, d, device=DEV, generator=g)
+    q[:, :, 45] *= 1e-39
+    lo = torch.full((8,), 5, device=DEV, dtype=torch.int32)
+    hi = torch.full((8,), T - 13, device=DEV, dtype=torch.int32)
+    refs = [exact(e, q, True, lo, hi, end) for end in (0, 80)]
+    assert float(refs[1][:, :, :40].abs().max()) == 0.0
+    st.vnorm.view(8, 8, -1)[:, :, :5] = math.inf
+    st.vnorm.view(8, 8, -1)[:, :, T - 13:T] = math.nan
+    st.knorm.view(8, 8, -1)[:, :, T - 13:T] = math.nan
+    for end, ref in zip((0, 80), refs):
+        out = e.attention(q, causal=True, kv_start=lo, kv_end=hi, q_end=end)
+        check(out, ref)
+        check(out[:, :, 45], ref[:, :, 45])   # uniform weights
+        assert not out[:, :, (ref == 0).all(-1).all(0).all(0)].any()
