@@ -737,9 +737,10 @@ extern "C" int qkv_compress_mfma(int32_t mode, int32_t in_dtype, const void* x, 
   const int64_t ntiles = (n + kTok - 1) / kTok;
   const dim3 grid(append_blocks(ntiles));
   const int xt = in_dtype == QKV_F32 ? 2 : in_dtype == QKV_F16 ? 1 : 0;
+  const int vec = qkv_aligned(codes, 16) && (!ip || qkv_aligned(qjl, 16));
 #define QKV_C(LV, IPV, XTV, DD)                                                                 \
   hipLaunchKernelGGL((compress_mfma<LV, IPV, XTV, DD>), grid, dim3(kThreads), 0, s, x, n,      \
-                     ntiles, pi, signs, h, codes, qjl, norms)
+                     ntiles, pi, signs, h, vec, codes, qjl, norms)
 #define QKV_CX(LV, IPV, DD)        \
   do {                             \
     if (xt == 2)                   \

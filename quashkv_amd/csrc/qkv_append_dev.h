@@ -977,123 +977,111 @@ __global__ __launch_bounds__(kThreads, 2) void append_kmix_mfma(
 // MSEQuantizer.compress / InnerProductQuantizer.compress and fused_compress_*
 // (quashkv/quantizer.py:113-131,211-242, quashkv/triton_kernels/compress.py:
 // 210-303) on the MFMA: n rows of dimension D into one uint8 code (and, IP,
-// one QJL bit) per coordinate, row-major, and the fp32 norms.  The rotation, search and tie rules are append_k_mfma's
-// (tokens x coordinates); IP searches the fine list (L = MB + 1 levels), MSE
-// the boundaries (L = bits levels).  A lane's code byte lands beside its
-// 31 neighbours' (32 coordinates of one row per half-wave).
+// one QJL bit) per coordinate, row-major, and the fp32 norms.  The rotation,
+// orientation and tie rules are append_k_mfma's (coordinates x tokens): IP
+// searches the fine list (L = MB + 1 levels), MSE the boundaries (L = bits
+// levels).  A lane holds 16 consecutive coordinates of its token per block, one
+// 16-byte store of codes (and of QJL bits); tokens x coordinates gave a byte
+// store per value, 64 or 128 a tile (200,003 fp32 rows, d = 128, IP: 61.1 us, now
+// 52.6, 2.9 TB/s).  A wave's registers hold the rows of one tile: its loads do not
+// overlap the tile before.  vec: codes and qjl 16-byte aligned.
 template <int L, bool IP, int XT, int D>
 __global__ __launch_bounds__(kThreads, 4) void compress_mfma(
     const void* __restrict__ xin, int64_t n, int64_t ntiles, const float* __restrict__ pi,
-    const float* __restrict__ signs, Half lst, uint8_t* __restrict__ codes,
+    const float* __restrict__ signs, Half lst, int vec, uint8_t* __restrict__ codes,
     uint8_t* __restrict__ qjl, float* __restrict__ norms) {
   constexpr bool F16 = XT != 0, F32 = XT == 2;
   constexpr int NP = (1 << (L - 1)) - 1;  // positive half of the searched list
   constexpr int NBK = D / 32, NKS = D / 16;
+  static_assert(kHalves == 1, "one token per lane");
   __shared__ uint4 frag[frag_n<D>()];
-  __shared__ float4 inv_s[kWaves][kTok / 4];
-  stage_pi<F16, D>(frag, pi, F16 ? kPScaleF16 : 1.f);
+  stage_pi<F16, D, true>(frag, pi, F16 ? kPScaleF16 : 1.f);
   __syncthreads();
 
-  const int lane = threadIdx.x & 63, li = lane & 31, wv = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, li = lane & 31, hh = lane >> 5, wv = threadIdx.x >> 6;
   uint32_t lv[NP > 0 ? NP : 1];
 #pragma unroll
   for (int i = 0; i < NP; ++i) lv[i] = in_vgpr(lst.t[i]);
-  uint32_t cx[NBK];  // IP: 1 where S >= 0 (the centroid level counts c <= y there)
-  uint32_t neg[NBK];  // IP: 1 where S < 0
+  // IP, per block: bits v of this lane half's coordinates 32 b + 16 hh + v, 1 where
+  // S < 0 (the bit's flip; where S >= 0 the centroid level counts c <= y)
+  uint32_t neg[NBK];
 #pragma unroll
   for (int b = 0; b < NBK; ++b) {
-    const bool ng = IP && signs[32 * b + li] < 0.f;
-    cx[b] = ng ? 0u : 1u;
-    neg[b] = ng ? 1u : 0u;
+    neg[b] = 0;
+    if constexpr (IP)
+      neg[b] = (static_cast<uint32_t>(lanes_where(signs[32 * b + li] < 0.f)) >> (16 * hh)) & 0xffffu;
   }
   const float iscale = F16 ? 1.f / kPScaleF16 : 1.f;
   const int64_t wstep = int64_t(gridDim.x) * kWaves;
+  auto put = [&](uint8_t* to, const uint32_t* w) {
+    if (vec) {
+      *reinterpret_cast<uint4*>(to) = make_uint4(w[0], w[1], w[2], w[3]);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) to[i] = static_cast<uint8_t>(w[i >> 2] >> (8 * (i & 3)));
+    }
+  };
 
   for (int64_t tile = int64_t(blockIdx.x) * kWaves + wv; tile < ntiles; tile += wstep) {
     const int64_t s0 = tile * kTok;
     const int nv = static_cast<int>(min<int64_t>(kTok, n - s0));
-    uint4 xf[kHalves][NKS];
-    uint4 xl[kHalves][F32 ? NKS : 1];  // fp32 rows: the low fp16 parts
-    float nrm[kHalves];
+    const int64_t srow = s0 + min(li, nv - 1);  // this lane's token row (clamped)
+    uint4 xf[1][NKS];
+    uint4 xl[1][F32 ? NKS : 1];  // fp32 rows: the low fp16 parts
+    float nrm[1];
     if constexpr (F32) {
-      const float* row[kHalves];
-#pragma unroll
-      for (int tt = 0; tt < kHalves; ++tt)
-        row[tt] = static_cast<const float*>(xin) + (s0 + min(32 * tt + li, nv - 1)) * D;
+      const float* row[1] = {static_cast<const float*>(xin) + srow * D};
       load_x_f32<NKS>(xf, xl, nrm, row, lane);
     } else {
-      const uint16_t* row[kHalves];
-#pragma unroll
-      for (int tt = 0; tt < kHalves; ++tt)
-        row[tt] = static_cast<const uint16_t*>(xin) + (s0 + min(32 * tt + li, nv - 1)) * D;
+      const uint16_t* row[1] = {static_cast<const uint16_t*>(xin) + srow * D};
       load_x<NKS>(xf, row, lane);
+      float ss = 0.f;
 #pragma unroll
-      for (int tt = 0; tt < kHalves; ++tt) {
-        float ss = 0.f;
-#pragma unroll
-        for (int s = 0; s < NKS; ++s) ss = sumsq<F16>(xf[tt][s], ss);
-        ss += __shfl_xor(ss, 32, 64);
-        nrm[tt] = fmaxf(sqrtf(ss), 1e-8f);
-      }
+      for (int s = 0; s < NKS; ++s) ss = sumsq<F16>(xf[0][s], ss);
+      ss += __shfl_xor(ss, 32, 64);
+      nrm[0] = fmaxf(sqrtf(ss), 1e-8f);
     }
-    float* invw = reinterpret_cast<float*>(&inv_s[wv][0]);
-#pragma unroll
-    for (int tt = 0; tt < kHalves; ++tt) {
-      if (lane < 32) {
-        if (32 * tt + li < nv) norms[s0 + 32 * tt + li] = nrm[tt];
-        if (!F32) invw[32 * tt + li] = iscale / nrm[tt];
-      }
-    }
-    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this wave's LDS writes landed
-    __builtin_amdgcn_wave_barrier();
+    if (lane < 32 && li < nv) norms[s0 + li] = nrm[0];
+    // (fp32 rows: scaled before the rotation)
+    const float iv = F32 ? 1.f / 65536.f : iscale / nrm[0];
 
     static_for<NBK>([&](auto nc) {  // coordinates 32 b .. 32 b + 31
       constexpr int b = decltype(nc)::value;
       __builtin_amdgcn_sched_barrier(0);
-      qkv_f32x16 acc[kHalves] = {};
+      qkv_f32x16 acc = {};
 #pragma unroll
       for (int s = 0; s < NKS; ++s)
 #pragma unroll
         for (int sp2 = 0; sp2 < 2; ++sp2) {
-          const uint4 bf = frag[((b * NKS + s) * 2 + sp2) * 64 + lane];
-#pragma unroll
-          for (int tt = 0; tt < kHalves; ++tt) {
-            acc[tt] = mma<F16>(xf[tt][s], bf, acc[tt]);
-            if (F32 && sp2 == 0) acc[tt] = mma<F16>(xl[tt][F32 ? s : 0], bf, acc[tt]);
-          }
+          const uint4 af = frag[((b * NKS + s) * 2 + sp2) * 64 + lane];
+          acc = mma<F16>(af, xf[0][s], acc);
+          if (F32 && sp2 == 0) acc = mma<F16>(af, xl[0][F32 ? s : 0], acc);
         }
+      // (opaque: the 16 flips, as invariants of the tile loop, took 56 registers to scratch)
+      if constexpr (IP) asm volatile("" : "+v"(neg[b]));
+      uint32_t cw[4], qw[4];  // four values a dword
 #pragma unroll
-      for (int tt = 0; tt < kHalves; ++tt) {
-        float4 iv4[4];
-        if constexpr (!F32) {
+      for (int j = 0; j < 4; ++j) {
+        uint32_t f = 0;
 #pragma unroll
-          for (int a = 0; a < 4; ++a) iv4[a] = inv_s[wv][8 * tt + 2 * a + (lane >> 5)];
+        for (int e = 0; e < 4; ++e) {
+          const int v = 4 * j + e;
+          const uint32_t cx = IP ? ((neg[b] >> v) & 1u) ^ 1u : 0u;
+          f |= search_sym_count<L, IP>(acc[v] * iv, lv, cx) << (8 * e);
         }
-        // this lane's first token 32 tt + 4 (l >> 5) at coordinate 32 b + (l & 31); the
-        // others sit at fixed offsets from it
-        const int64_t o0 = (s0 + 32 * tt + 4 * (lane >> 5)) * D + 32 * b + li;
-        uint8_t* cb = codes + o0;
-        uint8_t* qb = IP ? qjl + o0 : nullptr;
-        const int tk0 = 32 * tt + 4 * (lane >> 5);
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          float iv = 1.f / 65536.f;  // fp32 rows: scaled before the rotation
-          if constexpr (!F32) {
-            const float4 q4 = iv4[v >> 2];
-            iv = (v & 3) == 0 ? q4.x : (v & 3) == 1 ? q4.y : (v & 3) == 2 ? q4.z : q4.w;
-          }
-          // token tk0 + 8 (v >> 2) + (v & 3)
-          const int dt = 8 * (v >> 2) + (v & 3);
-          const uint32_t f = search_sym_count<L, IP>(acc[tt][v] * iv, lv, cx[b]);
-          if (tk0 + dt < nv) {
-            if constexpr (IP) {
-              cb[dt * D] = static_cast<uint8_t>(f >> 1);
-              qb[dt * D] = static_cast<uint8_t>((f & 1u) ^ neg[b]);
-            } else {
-              cb[dt * D] = static_cast<uint8_t>(f);
-            }
-          }
+        if constexpr (IP) {
+          cw[j] = (f >> 1) & 0x7f7f7f7fu;
+          // bit e of the block's flips into byte e
+          const uint32_t fl = (((neg[b] >> (4 * j)) & 15u) * 0x00204081u) & 0x01010101u;
+          qw[j] = (f & 0x01010101u) ^ fl;
+        } else {
+          cw[j] = f;
         }
+      }
+      if (li < nv) {
+        const int64_t at = srow * D + 32 * b + 16 * hh;
+        put(codes + at, cw);
+        if constexpr (IP) put(qjl + at, qw);
       }
     });
   }

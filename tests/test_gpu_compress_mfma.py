@@ -171,3 +171,25 @@ def test_index_add_fp32_vs_oracle(d):
         assert rate <= 2e-5 and step <= 1, (rate, step)
     got, ref = idx._norms[:n].cpu().double(), on.double()
     assert float(((got - ref).abs() / ref).max()) <= 2e-6
+
+
+@pytest.mark.parametrize("d", [128, 96, 64])
+@pytest.mark.parametrize("n,off", [(8, 1), (31, 4), (33, 8), (4097, 1)])
+def test_compress_unaligned_outputs(d, n, off):
+    """Outputs that 16-byte stores cannot take, and ragged last tiles: the same bytes,
+    and none beside them."""
+    x = _x(n, d, torch.float32, n).to(DEV)
+    q = Q.InnerProductQuantizer(d, total_bits=4, seed=3, device=DEV)
+    mq = q.mse_quantizer
+    c, b, nrm = q.compress(x)
+    bufs = [torch.full((n * d + 32,), 255, dtype=torch.uint8, device=DEV) for _ in range(3)]
+    outs = [t[off:off + n * d].view(n, d) for t in bufs]
+    got = torch.empty(n, dtype=torch.float32, device=DEV)
+    compress_into(N.QKV_MODE_IP, x, mq.Pi, mq.codebook.boundaries, mq.codebook.centroids, 3,
+                  q.S, outs[0], outs[1], got, packed=False)
+    compress_into(N.QKV_MODE_MSE, x, mq.Pi, mq.codebook.boundaries, mq.codebook.centroids, 3,
+                  None, outs[2], None, got, packed=False)
+    assert torch.equal(outs[0], c) and torch.equal(outs[1], b) and torch.equal(got, nrm)
+    assert _mismatch(outs[2], c)[1] <= 1
+    for t in bufs:
+        assert (t[:off] == 255).all() and (t[off + n * d:] == 255).all()
