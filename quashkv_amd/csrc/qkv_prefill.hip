@@ -659,21 +659,27 @@ __global__ __launch_bounds__(kThr, 2) void prefill(PreArgs A, KVLayers kv) {
       for (int r = 0; r < 16; ++r) O[ct][r] = O[ct][r] * f1 + mg[64 * (16 * ct + r)] * f2;
   }
 
-  // ---- partials: O~ (rotated, unnormalised) and (m, l) of the split
+  // ---- partials of the split: O~ / l (rotated) and (m, l) with the weights' sum in m,
+  // so that l is 1 as nearly as m's rounding allows: mref holds log2 |v|, and the raw l
+  // of large norms (~64 / |v|) would meet the merge's floor of 1e-8
   if (A.n_splits > 1) {
     const int64_t row = (int64_t(split) * A.BH + bh) * A.R + int64_t(g) * A.Q + qi;
+    const float e2 = mref - 6.f;
+    const float m = (e2 + __builtin_amdgcn_logf(l)) * 0.69314718055994531f;
+    // 2^(e2 - m log2 e), log2 e in two parts: 1 / l
+    const float f =
+        __builtin_amdgcn_exp2f(fmaf(-m, 1.92596299e-8f, fmaf(-m, 1.44269502f, e2)));
+    const float fo = l > 0.f ? f * A.vl.inv : 0.f;
     if (live && th == 0) {
 #pragma unroll
       for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
         for (int r = 0; r < 16; r += 4)
           *reinterpret_cast<float4*>(A.part_o + row * D + 32 * ct + 8 * (r >> 2) + 4 * h) =
-              make_float4(O[ct][r] * A.vl.inv, O[ct][r + 1] * A.vl.inv, O[ct][r + 2] * A.vl.inv,
-                          O[ct][r + 3] * A.vl.inv);
+              make_float4(O[ct][r] * fo, O[ct][r + 1] * fo, O[ct][r + 2] * fo, O[ct][r + 3] * fo);
       if (h == 0) {
-        A.part_ml[row * 2] =
-            l > 0.f ? (mref - 6.f) * 0.69314718055994531f : -INFINITY;
-        A.part_ml[row * 2 + 1] = l;
+        A.part_ml[row * 2] = l > 0.f ? m : -INFINITY;
+        A.part_ml[row * 2 + 1] = l > 0.f ? l * f : 0.f;
       }
     }
     return;

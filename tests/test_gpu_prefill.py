@@ -198,3 +198,20 @@ def test_prefill_extremes(d, T):
         check(out, ref)
         check(out[:, :, 45], ref[:, :, 45])   # uniform weights
         assert not out[:, :, (ref == 0).all(-1).all(0).all(0)].any()
+
+
+@pytest.mark.parametrize("d,splits", [(128, 1), (128, 4), (96, 3), (64, 4)])
+def test_prefill_split_large_value_norms(d, splits):
+    """Value norms to 1e12 (and 1e-12) over several splits: the merge's floor on the
+    weights' sum is no part of the result."""
+    e, g = filled(8, 8, 700, d, 3, 3, 21, dtype=torch.float32)
+    q = torch.randn(8, 32, 60, d, device=DEV, generator=g)
+    kq, vq = e.key_quantizer, e.value_quantizer
+    e._store.vnorm *= torch.tensor([1e12, 1e-12] * 4, device=DEV)[:, None]
+    ref = exact(e, q, True)
+    out = attention_store(q, e._store, 700, kq.mse_quantizer.Pi,
+                          kq.mse_quantizer.codebook.centroids_host,
+                          vq.codebook.centroids_host, kq.S, kq.qjl_scale, causal=True,
+                          n_splits=splits)
+    for h in range(8):   # one norm each
+        check(out[:, 4 * h:4 * h + 4], ref[:, 4 * h:4 * h + 4])
