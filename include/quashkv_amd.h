@@ -308,11 +308,14 @@ int qkv_vtiles_unpack(const uint32_t* src, int64_t groups, int64_t S, int32_t d,
  * kbits <= 2 run on the integer-MFMA kernel; other shapes on a VALU kernel.
  * ---------------------------------------------------------------------- */
 
-/* Split-K count the library would use for a decode-attention call. */
+/* Split-K count the library would use for a decode-attention call.  (A call of
+ * many query rows that the prefill kernel takes runs, at this count, as many
+ * splits of its own as pay and the workspace holds; any other count is kept.) */
 int32_t qkv_attention_splits(int32_t B, int32_t Hq, int32_t Hkv, int32_t Q,
                              int32_t d, int64_t T);
 
-/* Workspace bytes qkv_decode_attention needs for `n_splits` splits. */
+/* Workspace bytes qkv_decode_attention uses for `n_splits` splits (with 48 or
+ * more query rows per kv head: room for the prefill kernel's own splits). */
 int64_t qkv_attention_workspace_bytes(int32_t B, int32_t Hq, int32_t Hkv,
                                       int32_t Q, int32_t d, int32_t n_splits);
 

@@ -2220,8 +2220,8 @@ int launch_fused(const QLayers& ql, const KVLayers& kv, const OutLayers& ol, int
 
 // ------------------------------------------------------------ C ABI
 
-int combine_layers(const OutLayers& ol, int nl, int32_t B, int32_t Hq, int32_t Hkv, int32_t Q,
-                   int32_t d, int32_t out_dtype, void* workspace, int64_t ws_bytes,
+int launch_combine(const OutLayers& ol, int nl, int32_t B, int32_t Hq, int32_t Hkv, int32_t Q,
+                   int32_t d, int32_t out_dtype, const float* po, const float* pml,
                    int32_t n_splits, hipStream_t s);
 
 // Splits of the decode kernels (4 or 8 query rows per workgroup).
@@ -2243,17 +2243,14 @@ static int32_t decode_splits(int32_t B, int32_t Hq, int32_t Hkv, int32_t Q, int3
 }
 
 // Whether the prefill kernel is the faster one for R query rows in each of bh
-// (sequence, kv head) groups over T keys: both kernels' times in us as measured
-// (rounds of the chip's workgroups times their steps; fixed part; the merge of
-// splits).  E.g. d = 128, 8 groups: 48 rows over 256 keys 19 against 28 us, over
+// (sequence, kv head) groups over T keys, ds splits of the decode kernels against
+// ps of its own: both kernels' times in us as measured (rounds of the chip's
+// workgroups times their steps; fixed part; the merge of splits).  E.g. d = 128, 8 groups: 48 rows over 256 keys 19 against 28 us, over
 // 8192 keys 51 against 37; 256 rows over 2048 keys 42 against 39; 8192 rows over
 // 2048 keys 1052 against 144.
-static bool prefill_pays(int32_t B, int32_t Hq, int32_t Hkv, int32_t Q, int32_t d, int64_t T) {
-  const int R = (Hq / Hkv) * Q;
-  if (R < kPrefillMinRows || !qkv_d_ok(d)) return false;
-  const int64_t bh = int64_t(B) * Hkv, ncu = qkv_num_cus();
+static bool prefill_pays(int64_t bh, int R, int32_t d, int64_t T, int ds, int ps) {
+  const int64_t ncu = qkv_num_cus();
   auto rounds = [&](int64_t wgs) { return static_cast<double>((wgs + ncu - 1) / ncu); };
-  const int ds = decode_splits(B, Hq, Hkv, Q, d, T);
   double dec;
   if (d == 64) {  // decode_small: 8 rows per workgroup, three workgroups per CU
     dec = 12.0 + 2.7e-5 * double(bh * ((R + 7) / 8)) * double(T);
@@ -2262,7 +2259,6 @@ static bool prefill_pays(int32_t B, int32_t Hq, int32_t Hkv, int32_t Q, int32_t 
           (11.0 + 2.31 / 512.0 * double(T) / ds);
   }
   dec += ds > 1 ? 5.0 : 0.0;
-  const int ps = qkv_prefill_splits(bh, R, d, T);
   const double step = d == 128 ? 4.4 : d == 96 ? 3.2 : 2.0;  // per 64 tokens
   const double r = rounds(bh * ((R + 127) / 128) * ps);
   const double pre = 2.0 + r * (8.0 + step * double((T + 64 * ps - 1) / (64 * ps))) +
@@ -2273,50 +2269,66 @@ static bool prefill_pays(int32_t B, int32_t Hq, int32_t Hkv, int32_t Q, int32_t 
 extern "C" int32_t qkv_attention_splits(int32_t B, int32_t Hq, int32_t Hkv, int32_t Q,
                                         int32_t d, int64_t T) {
   if (B <= 0 || Hkv <= 0 || Hq <= 0 || Q <= 0 || T <= 0) return 1;
-  if (prefill_pays(B, Hq, Hkv, Q, d, T))
-    return qkv_prefill_splits(int64_t(B) * Hkv, (Hq / Hkv) * Q, d, T);
   return decode_splits(B, Hq, Hkv, Q, d, T);
 }
 
-// The prefill kernel's calls: one layer, codebooks it takes.  Its splits follow
-// its own rule (128 rows per workgroup), so a call it would have had but that
-// stays on the decode kernels has them cut to theirs.
-static bool use_prefill(int32_t B, int32_t Hq, int32_t Hkv, int32_t Q, int32_t d, int64_t T,
-                        int32_t kbits, int32_t vbits, const float* kcent, const float* vcent,
-                        float qjl_scale, int64_t t_stride) {
-  return prefill_pays(B, Hq, Hkv, Q, d, T) && t_stride % 64 == 0 &&
-         qkv_prefill_ok(d, kbits, vbits, kcent, vcent, qjl_scale);
-}
-static int clamp_splits(int32_t B, int32_t Hq, int32_t Hkv, int32_t Q, int32_t d, int64_t T,
-                        int n_splits) {
-  if (!prefill_pays(B, Hq, Hkv, Q, d, T)) return n_splits;
-  return std::min<int>(n_splits, decode_splits(B, Hq, Hkv, Q, d, T));
+// Bytes of one split's partials (O~, then (m, l)).
+static int64_t split_bytes(int64_t bh, int R, int d) { return bh * R * (int64_t(d) * 4 + 8); }
+
+// The prefill kernel's calls: one layer, codebooks it takes.  The caller's split
+// count is the decode kernels' (qkv_attention_splits, which the three-call form
+// and the layer and mixed-key entries run as it is); prefill needs nothing else
+// of the workspace, so it fills that with as many splits as its own rule (128
+// rows per workgroup) asks for.  A count of the caller's own is kept.
+// 0: the call stays on the decode kernels.
+static int prefill_count(int32_t B, int32_t Hq, int32_t Hkv, int32_t Q, int32_t d, int64_t T,
+                         int32_t kbits, int32_t vbits, const float* kcent, const float* vcent,
+                         float qjl_scale, int64_t t_stride, int64_t ws_bytes, int n_splits) {
+  const int R = (Hq / Hkv) * Q;
+  if (R < kPrefillMinRows || t_stride % 64 != 0) return 0;
+  const int64_t bh = int64_t(B) * Hkv;
+  const int ds = decode_splits(B, Hq, Hkv, Q, d, T);
+  const int own = static_cast<int>(std::max<int64_t>(
+      1, std::min<int64_t>(qkv_prefill_splits(bh, R, d, T), ws_bytes / split_bytes(bh, R, d))));
+  if (!prefill_pays(bh, R, d, T, ds, own) ||
+      !qkv_prefill_ok(d, kbits, vbits, kcent, vcent, qjl_scale))
+    return 0;
+  return n_splits == ds ? own : n_splits;
 }
 static int run_prefill(const void* q, int32_t q_dtype, const KVLayers& kv, int64_t t_stride,
                        int64_t T, int32_t B, int32_t Hq, int32_t Hkv, int32_t Q, int32_t d,
                        int32_t kbits, int32_t vbits, const float* pi, const float* kcent,
                        const float* vcent, const float* signs, float qjl_scale, float scale,
-                       int32_t causal, void* out, int32_t out_dtype, void* workspace,
-                       int64_t ws_bytes, int32_t n_splits, hipStream_t s) {
+                       int32_t causal, void* out, int32_t out_dtype, void* workspace, int splits,
+                       hipStream_t s) {
   QKV_REQUIRE(qkv_aligned(pi, 16) && qkv_aligned(kv.kst[0], 4) && qkv_aligned(kv.vst[0], 4),
               "pi must be 16-byte and the store 4-byte aligned");
-  const WsLayout L = ws_layout(B, Hkv, (Hq / Hkv) * Q, d, n_splits);
+  const int R = (Hq / Hkv) * Q;
+  float* po = static_cast<float*>(workspace);
+  float* pml = po + int64_t(splits) * B * Hkv * R * d;
   QkvPrefillArgs a{q,    q_dtype, kv,    t_stride,  T,     B,      Hq,  Hkv,       Q,
                    d,    kbits,   vbits, pi,        kcent, vcent,  signs, qjl_scale, scale,
-                   causal, out,   out_dtype, n_splits, at<float>(workspace, L.po),
-                   at<float>(workspace, L.pml)};
+                   causal, out,   out_dtype, splits, po, pml};
   const int st = qkv_prefill(a, s);
-  if (st != QKV_OK || n_splits == 1) return st;
+  if (st != QKV_OK || splits == 1) return st;
   OutLayers ol{};
   ol.pi[0] = pi;
   ol.out[0] = out;
-  return combine_layers(ol, 1, B, Hq, Hkv, Q, d, out_dtype, workspace, ws_bytes, n_splits, s);
+  return launch_combine(ol, 1, B, Hq, Hkv, Q, d, out_dtype, po, pml, splits, s);
 }
 
+// The decode kernels' layout for n_splits, and from kPrefillMinRows rows up room
+// for the prefill kernel's own splits (16 MiB at most, so that what the
+// no-allocation form takes is what its array holds; the CUs times 128 rows are 17 MB).
 extern "C" int64_t qkv_attention_workspace_bytes(int32_t B, int32_t Hq, int32_t Hkv, int32_t Q,
                                                  int32_t d, int32_t n_splits) {
   if (B <= 0 || Hkv <= 0 || Hq <= 0 || Q <= 0 || d <= 0 || n_splits <= 0) return -1;
-  return ws_layout(B, Hkv, (Hq / Hkv) * Q, d, n_splits).total;
+  const int R = (Hq / Hkv) * Q;
+  const int64_t need = ws_layout(B, Hkv, R, d, n_splits).total;
+  if (R < kPrefillMinRows || !qkv_d_ok(d)) return need;
+  const int64_t bh = int64_t(B) * Hkv;
+  const int64_t room = qkv_prefill_splits(bh, R, d, INT64_MAX) * split_bytes(bh, R, d);
+  return std::max(need, std::min<int64_t>(room, QKV_NOALLOC_SCRATCH_BYTES));
 }
 
 extern "C" int32_t qkv_attention_path(int32_t d, int32_t kbits, int32_t vbits,
@@ -2533,15 +2545,20 @@ int combine_layers(const OutLayers& ol, int nl, int32_t B, int32_t Hq, int32_t H
     QKV_REQUIRE(ol.pi[l] && ol.out[l], "null pointer");
     QKV_REQUIRE(qkv_aligned(ol.pi[l], 16), "pi must be 16-byte aligned");
   }
+  const WsLayout L = ws_layout(B * nl, Hkv, (Hq / Hkv) * Q, d, n_splits);
+  return launch_combine(ol, nl, B, Hq, Hkv, Q, d, out_dtype, at<float>(workspace, L.po),
+                        at<float>(workspace, L.pml), n_splits, s);
+}
+
+int launch_combine(const OutLayers& ol, int nl, int32_t B, int32_t Hq, int32_t Hkv, int32_t Q,
+                   int32_t d, int32_t out_dtype, const float* po, const float* pml,
+                   int32_t n_splits, hipStream_t s) {
   const int R = (Hq / Hkv) * Q;
-  const WsLayout L = ws_layout(B * nl, Hkv, R, d, n_splits);
   const int64_t nrl = int64_t(B) * Hkv * R;  // rows per layer
   // few rows: one per workgroup (more workgroups over the splits); many rows:
   // four per workgroup (each Pi load serves four)
   const bool wide = nrl * nl < int64_t(kRowsC) * qkv_num_cus();
   const dim3 cgrid(static_cast<int>(wide ? nrl : (nrl + kRowsC - 1) / kRowsC), nl);
-  const float* po = at<float>(workspace, L.po);
-  const float* pml = at<float>(workspace, L.pml);
   switch (d) {
 #define QKV_CASE(DD)                                                                          \
   case DD:                                                                                    \
@@ -2625,12 +2642,12 @@ int decode_attention_impl(const void* q, int32_t q_dtype, const uint8_t* kstore,
   kv.khi = kr.khi;
   kv.cbase = kr.cbase;
   auto s = static_cast<hipStream_t>(stream);
-  if (use_prefill(B, Hq, Hkv, Q, d, T, kbits, vbits, kcent_host, vcent_host, qjl_scale,
-                  t_stride))
+  const int ps = prefill_count(B, Hq, Hkv, Q, d, T, kbits, vbits, kcent_host, vcent_host,
+                               qjl_scale, t_stride, ws_bytes, n_splits);
+  if (ps > 0)
     return run_prefill(q, q_dtype, kv, t_stride, T, B, Hq, Hkv, Q, d, kbits, vbits, pi,
                        kcent_host, vcent_host, signs, qjl_scale, scale, causal, out, out_dtype,
-                       workspace, ws_bytes, n_splits, s);
-  n_splits = clamp_splits(B, Hq, Hkv, Q, d, T, n_splits);
+                       workspace, ps, s);
   const Tables tb = make_tables(kcent_host, kbits, vcent_host, vbits);
   if (d == 64 && tb.mfma_ok && t_stride % 64 == 0 && !kr.klo && !kr.khi && kr.cbase == 0) {
     // decode_small: one launch (plus combine_kernel with several splits)
@@ -2766,12 +2783,9 @@ extern "C" int qkv_decode_attention_noalloc(const void* q, int32_t q_dtype,
                                             int32_t n_splits, void* stream) {
   QKV_REQUIRE(B > 0 && Hq > 0 && Hkv > 0 && Q > 0 && Hq % Hkv == 0, "invalid shape");
   QKV_REQUIRE(n_splits >= 1 && n_splits <= 1024, "n_splits %d out of range", n_splits);
-  int64_t need = qkv_attention_workspace_bytes(B, Hq, Hkv, Q, d, n_splits);
-  QKV_REQUIRE(need > 0, "invalid shape");
-  // the prefill kernel's splits are a matter of speed only: as many as fit
-  while (need > int64_t(QKV_NOALLOC_SCRATCH_BYTES) && n_splits > 1 &&
-         prefill_pays(B, Hq, Hkv, Q, d, T))
-    need = qkv_attention_workspace_bytes(B, Hq, Hkv, Q, d, --n_splits);
+  QKV_REQUIRE(d > 0, "invalid shape");
+  // (the prefill kernel's own splits are as many as fit)
+  const int64_t need = ws_layout(B, Hkv, (Hq / Hkv) * Q, d, n_splits).total;
   QKV_REQUIRE(need <= int64_t(QKV_NOALLOC_SCRATCH_BYTES),
               "qkv_decode_attention_noalloc: this call needs %lld workspace bytes, more than "
               "the %lld-byte scratch array (use qkv_decode_attention with a workspace)",
@@ -2826,12 +2840,12 @@ extern "C" int qkv_paged_decode_attention(
   kv.pmax = pages_per_seq;
   kv.plg = plg;
   kv.npages = num_pages;
-  if (use_prefill(B, Hq, Hkv, Q, d, T, kbits, vbits, kcent_host, vcent_host, qjl_scale,
-                  t_stride))
+  const int ps = prefill_count(B, Hq, Hkv, Q, d, T, kbits, vbits, kcent_host, vcent_host,
+                               qjl_scale, t_stride, ws_bytes, n_splits);
+  if (ps > 0)
     return run_prefill(q, q_dtype, kv, t_stride, T, B, Hq, Hkv, Q, d, kbits, vbits, pi,
                        kcent_host, vcent_host, signs, qjl_scale, scale, causal, out, out_dtype,
-                       workspace, ws_bytes, n_splits, static_cast<hipStream_t>(stream));
-  n_splits = clamp_splits(B, Hq, Hkv, Q, d, T, n_splits);
+                       workspace, ps, static_cast<hipStream_t>(stream));
   {  // the kernels of the contiguous single call: decode_small at d = 64 with
      // key MSE bits <= 2, decode_fused otherwise
     QLayers ql{};
@@ -2901,7 +2915,6 @@ static int decode_layers(int32_t n_layers, const void* const* q, int32_t q_dtype
                   "bits <= 3, capacity a multiple of 64)");
     return QKV_E_UNSUPPORTED;
   }
-  n_splits = clamp_splits(B * n_layers, Hq, Hkv, Q, d, T, n_splits);
   QLayers ql{};
   KVLayers kv{};
   OutLayers ol{};
@@ -3017,7 +3030,6 @@ int kmixed_decode_impl(int kind, const void* q, int32_t q_dtype, const uint8_t* 
   }
   QKV_REQUIRE(qkv_aligned(pi_perm, 16) && qkv_aligned(pi_v, 16), "pi must be 16-byte aligned");
   QKV_REQUIRE(qkv_aligned(kstore, 4), "K rows must be 4-byte aligned");
-  n_splits = clamp_splits(B, Hq, Hkv, Q, d, T, n_splits);
   QLayers ql{};
   ql.q[0] = q;
   ql.pi[0] = pi_perm;

@@ -215,3 +215,54 @@ def test_prefill_split_large_value_norms(d, splits):
                           n_splits=splits)
     for h in range(8):   # one norm each
         check(out[:, 4 * h:4 * h + 4], ref[:, 4 * h:4 * h + 4])
+
+
+def _call(e, q, causal, form):
+    """qkv_decode_attention by its workspace, no-allocation or three-call form."""
+    st, kq, vq = e._store, e.key_quantizer, e.value_quantizer
+    mq = kq.mse_quantizer
+    B, Hq, Q, d = q.shape
+    T = e.total_tokens
+    L, s = N.lib(), N.stream(q.device)
+    kc = N.HostFloats(mq.codebook.centroids_host)
+    vc = N.HostFloats(vq.codebook.centroids_host)
+    out = torch.full((B, Hq, Q, d), math.nan, device=DEV)
+    ns = L.qkv_attention_splits(B, Hq, st.H, Q, d, T)
+    ws = torch.empty(L.qkv_attention_workspace_bytes(B, Hq, st.H, Q, d, ns), dtype=torch.uint8,
+                     device=DEV)
+    qa = (q.data_ptr(), N.dtype_code(q.dtype))
+    kv = (st.kst.data_ptr(), st.knorm.data_ptr(), st.vst.data_ptr(), st.vnorm.data_ptr(),
+          st.capacity, T)
+    dims = (B, Hq, st.H, Q, d, st.mbits, st.vbits)
+    tail = (1.0 / math.sqrt(d), int(causal), out.data_ptr(), N.QKV_F32)
+    w = (ws.data_ptr(), ws.numel(), ns, s)
+    if form == "phases":
+        N.check(L.qkv_attention_prepare(*qa, *dims, mq.Pi.data_ptr(), kc.ptr, vc.ptr,
+                                        kq.S.data_ptr(), kq.qjl_scale, *w))
+        N.check(L.qkv_attention_run(*kv, *dims, mq.Pi.data_ptr(), kc.ptr, vc.ptr, *tail, *w))
+    else:
+        args = (*qa, *kv, *dims, mq.Pi.data_ptr(), kc.ptr, vc.ptr, kq.S.data_ptr(), kq.qjl_scale,
+                *tail)
+        if form == "noalloc":
+            N.check(L.qkv_decode_attention_noalloc(*args, ns, s))
+        else:
+            N.check(L.qkv_decode_attention(*args, *w))
+    return out
+
+
+@pytest.mark.parametrize("B,H,G,Q,d,T", [(8, 8, 4, 64, 64, 8192), (1, 8, 1, 128, 128, 8200),
+                                         (2, 4, 2, 64, 96, 4096)])
+def test_many_rows_by_every_form(B, H, G, Q, d, T):
+    """The split count of the library in the single call (the prefill kernel's own
+    splits, also where the no-allocation array holds fewer than it asks for) and in
+    the three-call form, whose kernels it is for."""
+    e, g = filled(B, H, T, d, 3, 3, 17)
+    q = torch.randn(B, H * G, Q, d, device=DEV, generator=g)
+    ref = exact(e, q, True)
+    a = _call(e, q, True, "workspace")
+    check(a, ref)
+    assert torch.equal(a, e.attention(q, causal=True))
+    check(_call(e, q, True, "phases"), ref)
+    rows = B * H * G * Q
+    if rows * (12 * d + 1552) < N.NOALLOC_SCRATCH_BYTES:
+        assert torch.equal(a, _call(e, q, True, "noalloc"))

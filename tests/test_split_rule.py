@@ -1,5 +1,6 @@
-"""Split counts of the fused decode where the row groups do not divide the CUs
-(256 without a device): no nearly empty last round of workgroups."""
+"""Split counts of the decode kernels (256 CUs without a device): of the fused one
+where the row groups do not divide the CUs, no nearly empty last round of
+workgroups; of many query rows, what the three-call form can run."""
 
 import pytest
 
@@ -16,3 +17,25 @@ from quashkv_amd import _native as N
 ])
 def test_splits_of_odd_group_counts(B, Hq, Hkv, d, T, splits):
     assert N.lib().qkv_attention_splits(B, Hq, Hkv, 1, d, T) == splits
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,Q,d,T,splits", [
+    (8, 32, 8, 64, 64, 8192, 4),      # split_mfma's scores fit LDS up to 2048 tokens a split
+    (1, 8, 8, 48, 64, 65536, 32),
+    (1, 8, 8, 256, 128, 2048, 1),     # 512 row groups: no splits, whatever the prefill kernel likes
+    (2, 8, 4, 64, 96, 4096, 1),
+])
+def test_splits_of_many_rows_serve_the_three_call_form(B, Hq, Hkv, Q, d, T, splits):
+    L = N.lib()
+    s = L.qkv_attention_splits(B, Hq, Hkv, Q, d, T)
+    assert s == splits
+    if d == 64:
+        assert -(-T // s) <= 2048
+    # room for the decode layout, and for the prefill kernel's splits within the
+    # no-allocation form's array
+    R = Hq // Hkv * Q
+    rows, ch = B * Hkv * R, B * Hkv * ((R + 3) // 4)
+    layout = rows * 8 * d + ch * (6 * 64 * 16 + 32) + s * rows * (4 * d + 8)
+    own = min(64, 256 // (B * Hkv * ((R + 127) // 128)))
+    room = min(N.NOALLOC_SCRATCH_BYTES, max(1, own) * rows * (4 * d + 8))
+    assert L.qkv_attention_workspace_bytes(B, Hq, Hkv, Q, d, s) == max(layout, room)
