@@ -812,7 +812,15 @@ void fill_levels(const float* cent, int bits, float s, Levels* lv) {
 struct PreLevels {
   Levels kl, vl;
   float ks;
+  bool fits;  // levels and QJL weight well inside f16's range at their scales
 };
+
+// Largest positive magnitude of a symmetric codebook (its upper half, in any order).
+float top_level(const float* cent, int bits) {
+  float top = 0.f;
+  for (int c = 1 << (bits - 1); c < 1 << bits; ++c) top = std::max(top, cent[c]);
+  return top;
+}
 
 // The levels of a (key, value) codebook pair: a pure function of its arguments,
 // 1024 candidate scales per codebook (~10 us), kept for the last pair per thread.
@@ -840,7 +848,7 @@ const PreLevels& levels_for(int d, int kbits, int vbits, const float* kc, const 
   if (!key_lo(d, kbits)) {
     m.lv.ks = best_scale(kp, 1 << (kbits - 1), fabsf(alpha), 0.1f);
   } else {
-    const float top = kp[(1 << (kbits - 1)) - 1];
+    const float top = top_level(kc, kbits);
     const float lo = alpha != 0.f ? fabsf(alpha) : top;
     int e;
     frexpf(top, &e);
@@ -850,7 +858,10 @@ const PreLevels& levels_for(int d, int kbits, int vbits, const float* kc, const 
     m.lv.ks = ldexpf(1.f / ma, 4 - e);
   }
   const float vs = vbits <= 2 ? best_scale(vp, 1 << (vbits - 1), 0.f, 0.f)
-                              : 16.f / vp[(1 << (vbits - 1)) - 1];
+                              : 16.f / top_level(vc, vbits);
+  auto in_f16 = [](float x) { return x <= 32768.f; };  // (false for NaN)
+  m.lv.fits = m.lv.ks > 0.f && vs > 0.f && in_f16(top_level(kc, kbits) * m.lv.ks) &&
+              in_f16(fabsf(alpha) * m.lv.ks) && in_f16(top_level(vc, vbits) * vs);
   fill_levels(kc, kbits, m.lv.ks, &m.lv.kl);
   fill_levels(vc, vbits, vs, &m.lv.vl);
   return m.lv;
@@ -883,10 +894,12 @@ bool qkv_prefill_ok(int d, int kbits, int vbits, const float* kcent, const float
                     float qjl_scale) {
   if (!qkv_d_ok(d) || kbits < 1 || kbits > 3 || vbits < 1 || vbits > 4) return false;
   if (!symmetric(kcent, kbits) || !symmetric(vcent, vbits)) return false;
-  // f16 range of the QJL weight at the key levels' scale
-  const float top = kcent[(1 << kbits) - 1], a = fabsf(qjl_scale);
+  // the QJL weight and the key levels within reach of one scale
+  const float top = top_level(kcent, kbits), a = fabsf(qjl_scale);
+  for (int c = 1 << (kbits - 1); c < 1 << kbits; ++c)
+    if (!(kcent[c] > 1e-2f * top)) return false;
   return a < 1e3f * top && (a == 0.f || a > 1e-4f * top) &&
-         kcent[1 << (kbits - 1)] > 1e-2f * top;
+         levels_for(d, kbits, vbits, kcent, vcent, qjl_scale).fits;
 }
 
 int qkv_prefill_splits(int64_t bh, int R, int d, int64_t T) {

@@ -31,7 +31,8 @@ def _need_gpu():
     N.lib()
 
 
-def exact(e, q, causal, lo=None, hi=None, q_end=0, signs=None, logits=False):
+def exact(e, q, causal, lo=None, hi=None, q_end=0, signs=None, logits=False, kcent=None,
+          vcent=None, qjl=None):
     b0 = e._cache[0]
     kc = torch.cat([b.mse_indices for b in e._cache], 2).long()
     vc = torch.cat([b.val_indices for b in e._cache], 2).long()
@@ -45,11 +46,13 @@ def exact(e, q, causal, lo=None, hi=None, q_end=0, signs=None, logits=False):
     B, Hq, Q, d = q.shape
     Hkv, T = kc.shape[1:3]
     G = Hq // Hkv
-    k = mq.codebook.centroids.double()[kc].repeat_interleave(G, 1)
+    table = lambda c, own: own if c is None else torch.tensor(c, device=q.device)  # noqa: E731
+    k = table(kcent, mq.codebook.centroids).double()[kc].repeat_interleave(G, 1)
     sg = ((2 * qs - 1) * S).repeat_interleave(G, 1)
-    v = (vq.codebook.centroids.double()[vc] * vn[..., None]).repeat_interleave(G, 1)
+    v = (table(vcent, vq.codebook.centroids).double()[vc] * vn[..., None]).repeat_interleave(G, 1)
     qr = q.double() @ mq.Pi.double().T
-    s = qr @ k.transpose(2, 3) + kq.qjl_scale * (qr.abs() @ sg.transpose(2, 3))
+    s = qr @ k.transpose(2, 3) + (kq.qjl_scale if qjl is None else qjl) * (
+        qr.abs() @ sg.transpose(2, 3))
     s = s * kn.repeat_interleave(G, 1)[:, :, None] / math.sqrt(d)
     top = float(s.abs().max())
     t = torch.arange(T, device=q.device)
@@ -266,3 +269,23 @@ def test_many_rows_by_every_form(B, H, G, Q, d, T):
     rows = B * H * G * Q
     if rows * (12 * d + 1552) < N.NOALLOC_SCRATCH_BYTES:
         assert torch.equal(a, _call(e, q, True, "noalloc"))
+
+
+@pytest.mark.parametrize("kb,vb,kc,vc,qjl", [
+    (3, 2, (0.0011, 0.1), None, 95.0),            # a QJL weight past f16 at the levels' scale
+    (3, 2, None, (1.0, 2e5), None),               # value levels likewise
+    (3, 3, (0.15, 0.05), (3e5, 0.9, 0.3, 1.0), None),   # levels in no order
+    (4, 4, (0.05, 0.2, 0.1, 0.15), (.4, .1, .3, .2, .8, .5, .7, .6), None),
+])
+def test_prefill_other_codebooks(kb, vb, kc, vc, qjl):
+    """Symmetric codebooks beyond the library's own, of the magnitudes given."""
+    e, g = filled(8, 8, 333, 128, kb, vb, 3)
+    e._store.knorm *= 0.01
+    q = torch.randn(8, 32, 40, 128, device=DEV, generator=g)
+    kq, vq = e.key_quantizer, e.value_quantizer
+    both = lambda m, own: [-x for x in m[::-1]] + list(m) if m else own   # noqa: E731
+    kc = both(kc, kq.mse_quantizer.codebook.centroids_host)
+    vc = both(vc, vq.codebook.centroids_host)
+    qjl = kq.qjl_scale if qjl is None else qjl
+    out = attention_store(q, e._store, 333, kq.mse_quantizer.Pi, kc, vc, kq.S, qjl, causal=True)
+    check(out, exact(e, q, True, kcent=kc, vcent=vc, qjl=qjl))
