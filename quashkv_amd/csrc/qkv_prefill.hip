@@ -486,9 +486,13 @@ __global__ __launch_bounds__(kThr, 2) void prefill(PreArgs A, KVLayers kv) {
     float* nm = reinterpret_cast<float*>(buf + C::OFF_N);
     if (wave < 2) {
       if (h == 0) {
-        nm[32 * wave + n] = wave == 0 ? r.nm * A.c0 : r.nm;
+        // a value norm that is not finite: weight 0 times 0 where the slot is masked, a
+        // reference of infinity (NaN out) for the rows that see it
+        const bool fin = wave == 0 || fabsf(r.nm) < INFINITY;
+        nm[32 * wave + n] = wave == 0 ? r.nm * A.c0 : fin ? r.nm : 0.f;
         // log2, from 2^-90 up: a row of zero norms alone keeps finite weights
-        if (wave == 1) nm[64 + n] = __builtin_amdgcn_logf(fmaxf(fabsf(r.nm), kMinNorm));
+        if (wave == 1)
+          nm[64 + n] = fin ? __builtin_amdgcn_logf(fmaxf(fabsf(r.nm), kMinNorm)) : INFINITY;
       }
     }
   };
@@ -678,8 +682,9 @@ __global__ __launch_bounds__(kThr, 2) void prefill(PreArgs A, KVLayers kv) {
           *reinterpret_cast<float4*>(A.part_o + row * D + 32 * ct + 8 * (r >> 2) + 4 * h) =
               make_float4(O[ct][r] * fo, O[ct][r + 1] * fo, O[ct][r + 2] * fo, O[ct][r + 3] * fo);
       if (h == 0) {
-        A.part_ml[row * 2] = l > 0.f ? m : -INFINITY;
-        A.part_ml[row * 2 + 1] = l > 0.f ? l * f : 0.f;
+        // (l NaN: no reference that the merge would leave out)
+        A.part_ml[row * 2] = l > 0.f ? m : l == 0.f ? -INFINITY : 0.f;
+        A.part_ml[row * 2 + 1] = l > 0.f ? l * f : l;
       }
     }
     return;

@@ -289,3 +289,26 @@ def test_prefill_other_codebooks(kb, vb, kc, vc, qjl):
     qjl = kq.qjl_scale if qjl is None else qjl
     out = attention_store(q, e._store, 333, kq.mse_quantizer.Pi, kc, vc, kq.S, qjl, causal=True)
     check(out, exact(e, q, True, kcent=kc, vcent=vc, qjl=qjl))
+
+
+@pytest.mark.parametrize("d,splits", [(64, 1), (128, 1), (128, 3)])
+def test_prefill_non_finite_norms_behind_the_mask(d, splits):
+    """Slots that are not finite: rows before them do not notice, rows that see them
+    are not finite either."""
+    T, Q = 700, 60
+    e, g = filled(8, 8, T, d, 3, 3, 23)
+    q = torch.randn(8, 32, Q, d, device=DEV, generator=g)
+    kq, vq = e.key_quantizer, e.value_quantizer
+    ref = exact(e, q, True)
+    for slot, bad in ((T - 20, math.inf), (T - 33, math.nan)):
+        norm = e._store.vnorm if bad == math.inf else e._store.knorm
+        norm[:, :, slot] = bad
+        if bad != math.inf:
+            e._store.vnorm[:, :, slot] = bad
+        out = attention_store(q, e._store, T, kq.mse_quantizer.Pi,
+                              kq.mse_quantizer.codebook.centroids_host,
+                              vq.codebook.centroids_host, kq.S, kq.qjl_scale, causal=True,
+                              n_splits=splits)
+        i = slot - (T - Q)   # the first query that sees it
+        check(out[:, :, :i], ref[:, :, :i])
+        assert not torch.isfinite(out[:, :, i:]).all(-1).any()
