@@ -370,7 +370,9 @@ int qkv_decode_attention_ranges(const void* q, int32_t q_dtype, const uint8_t* k
  * qkv_decode_attention without `workspace` / `ws_bytes`: the workspace is a
  * static device array of QKV_NOALLOC_SCRATCH_BYTES held by the library on
  * each GPU it runs on until the process ends.  A call whose workspace
- * (qkv_attention_workspace_bytes) exceeds that size returns QKV_E_INVALID.
+ * (qkv_attention_workspace_bytes; of 48 or more query rows per kv head, without
+ * the room for the prefill kernel's own splits, which are as many as fit)
+ * exceeds that size returns QKV_E_INVALID.
  * The library allocates nothing on this path.  Calls that overlap on one GPU
  * (different streams or threads) share the array and race; the last call's
  * contents stay in it. */

@@ -2318,8 +2318,7 @@ static int run_prefill(const void* q, int32_t q_dtype, const KVLayers& kv, int64
 }
 
 // The decode kernels' layout for n_splits, and from kPrefillMinRows rows up room
-// for the prefill kernel's own splits (16 MiB at most, so that what the
-// no-allocation form takes is what its array holds; the CUs times 128 rows are 17 MB).
+// for the prefill kernel's own splits (17 MB at most: the CUs times 128 rows).
 extern "C" int64_t qkv_attention_workspace_bytes(int32_t B, int32_t Hq, int32_t Hkv, int32_t Q,
                                                  int32_t d, int32_t n_splits) {
   if (B <= 0 || Hkv <= 0 || Hq <= 0 || Q <= 0 || d <= 0 || n_splits <= 0) return -1;
@@ -2327,8 +2326,7 @@ extern "C" int64_t qkv_attention_workspace_bytes(int32_t B, int32_t Hq, int32_t 
   const int64_t need = ws_layout(B, Hkv, R, d, n_splits).total;
   if (R < kPrefillMinRows || !qkv_d_ok(d)) return need;
   const int64_t bh = int64_t(B) * Hkv;
-  const int64_t room = qkv_prefill_splits(bh, R, d, INT64_MAX) * split_bytes(bh, R, d);
-  return std::max(need, std::min<int64_t>(room, QKV_NOALLOC_SCRATCH_BYTES));
+  return std::max(need, qkv_prefill_splits(bh, R, d, INT64_MAX) * split_bytes(bh, R, d));
 }
 
 extern "C" int32_t qkv_attention_path(int32_t d, int32_t kbits, int32_t vbits,

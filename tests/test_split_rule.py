@@ -31,11 +31,10 @@ def test_splits_of_many_rows_serve_the_three_call_form(B, Hq, Hkv, Q, d, T, spli
     assert s == splits
     if d == 64:
         assert -(-T // s) <= 2048
-    # room for the decode layout, and for the prefill kernel's splits within the
-    # no-allocation form's array
+    # room for the decode layout, and for the prefill kernel's splits
     R = Hq // Hkv * Q
     rows, ch = B * Hkv * R, B * Hkv * ((R + 3) // 4)
     layout = rows * 8 * d + ch * (6 * 64 * 16 + 32) + s * rows * (4 * d + 8)
     own = min(64, 256 // (B * Hkv * ((R + 127) // 128)))
-    room = min(N.NOALLOC_SCRATCH_BYTES, max(1, own) * rows * (4 * d + 8))
+    room = max(1, own) * rows * (4 * d + 8)
     assert L.qkv_attention_workspace_bytes(B, Hq, Hkv, Q, d, s) == max(layout, room)
