@@ -9,15 +9,20 @@
 // per 32 rows, one per 32-token half) and steps through 64 tokens at a time: the tile's codes become f16 levels
 // in LDS once, and the products run on v_mfma_f32_32x32x16_f16.
 //
-// Precision, against 64 bits no worse than the decode kernels' (6e-6 relative):
-//   * q~ = q Pi^T in three f16 products (hi hi + hi lo + lo hi, ~22 bits), kept
-//     as f16 hi + lo per row; both meet every key level;
-//   * key levels: one scale s brings the 1 or 2 magnitudes of a codebook (to ~2^-19)
-//     and the QJL weight, a tenth of them (to ~2^-15), near f16 values at once, by
-//     search over the 1024 mantissas of the first: 3 10^-6 of a score; codebooks of
-//     4 magnitudes, and d = 64, keep hi + lo;
-//   * softmax weights times |v| as f16 hi + lo (22 bits), value levels likewise.
-//   Sums are fp32 MFMA accumulators.
+// Precision: every f16 pair below is hi + lo, both rounded to nearest (24 bits).
+//   * q~ = q Pi^T in three f16 products (hi hi + hi lo + lo hi), kept as hi + lo per
+//     row; both meet every key level and the QJL weight;
+//   * key levels: hi + lo, with a scale at which the QJL weight is an f16 value.
+//     Codebooks of 1 magnitude, and of 2 at d >= 96, keep one f16 each: a scale s, by
+//     search over the 1024 mantissas of the first level, brings the second to 5e-7
+//     (1 magnitude: the QJL weight to 1e-7); what f16 then leaves of the QJL weight
+//     (~1e-4) is put back by one multiplication of the QJL term's sums;
+//   * softmax weights times |v| hi + lo, value levels likewise (1 magnitude: exact).
+//   Sums are fp32 MFMA accumulators.  Relative errors against 64 bits, N(0, 1) queries
+//   over 512 / 1500 keys: 0.5e-6 - 1.0e-6 / 0.7e-6 - 1.2e-6 (the decode kernels 1.1e-6 /
+//   1.5e-6 at d = 64 with up to 2 MSE bits, 6e-6 - 10e-6 otherwise); logits up to 100 -
+//   170: 1.1e-6 - 1.8e-6 (1.2e-6 - 23e-6); logits near 0, where the fp32 sums over the
+//   keys set it: 2.2e-7 - 2.6e-7 (1.8e-7 - 5.5e-7).
 //
 // Layout.  The score product is S^T = K Q^T (rows tokens, columns query rows),
 // so a lane owns one query row (lane & 31) and 16 of the 32 tokens: the softmax
@@ -58,7 +63,6 @@ __device__ __forceinline__ int64_t imax(int64_t a, int64_t b) { return a > b ? a
 
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef _Float16 v2h __attribute__((ext_vector_type(2)));
-typedef __fp16 v2fp __attribute__((ext_vector_type(2)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef uint32_t v4u __attribute__((ext_vector_type(4)));
 
@@ -86,6 +90,7 @@ struct PreArgs {
   const float* pi;
   const float* signs;
   float alpha;   // qjl_scale times the key levels' scale
+  float ae;      // alpha / f16(alpha) - 1 (0 unless PreCfg::AE)
   float c0;      // scale log2(e) / key levels' scale
   int causal;
   int64_t split_len;
@@ -105,10 +110,12 @@ __device__ __forceinline__ v16f mfma_h(v4u a, v4u b, v16f c) {
                                                 __builtin_bit_cast(v8h, b), c, 0, 0, 0);
 }
 
+typedef float v2f __attribute__((ext_vector_type(2)));
+
 __device__ __forceinline__ uint32_t pk(float a, float b) {
-  return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(a, b));
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((v2f{a, b}), v2h));
 }
-// x as f16 hi (truncated) + lo, two values per dword
+// x as f16 hi + lo, both rounded to nearest (24 bits, no bias), two values per dword
 __device__ __forceinline__ void split2(float a, float b, uint32_t& hi, uint32_t& lo) {
   hi = pk(a, b);
   const v2h h = __builtin_bit_cast(v2h, hi);
@@ -175,14 +182,15 @@ __device__ __forceinline__ void expand_unit(const uint32_t* w, int p, v4u th, v4
 }
 
 // Whether key levels keep f16 hi + lo.  At d = 64 the decode kernel's int8 scores
-// are good to ~1e-6 already, which single f16 levels (3.6e-6) are not.
+// are good to ~1e-6 already, and a product more costs less than at d = 128.
 __host__ __device__ constexpr bool key_lo(int d, int mb) { return mb >= 3 || (mb == 2 && d == 64); }
 
 template <int CT, int MB, int VB>
 struct PreCfg {
   static constexpr int D = 32 * CT;
   static constexpr int KK = 2 * CT;                 // 16-wide k steps of a d-long sum
-  static constexpr bool KLO = key_lo(32 * CT, MB), VLO = VB >= 3;
+  static constexpr bool KLO = key_lo(32 * CT, MB), VLO = VB >= 2;
+  static constexpr bool AE = MB == 2 && !KLO;       // the QJL weight's f16 error is mended
   static constexpr int KPW = (KK + 3) / 4;          // units of K and of V per thread and step
   static constexpr int SEG = KK * 1024;             // bytes of one operand image
   static constexpr int OFF_S = SEG * (KLO ? 2 : 1), OFF_V = OFF_S + SEG;
@@ -359,8 +367,8 @@ __global__ __launch_bounds__(kThr, 2) void prefill(PreArgs A, KVLayers kv) {
   }
 
   // QJL operand constants of this thread's K units: f16(alpha S_j), negated (a set
-  // bit flips the sign back); eps: what f16 leaves of them.  Signs other than +-1
-  // (more than 4e-5 of them left) take a third QJL product.
+  // bit flips the sign back); eps: what f16 and (1 + ae) leave of them.  Signs other
+  // than +-1 (more than 1e-6 of them left) take a third QJL product.
   const int w0 = (wave * KPW) >> 1;  // this thread's plane word, for K and for V
   const bool work = wave * KPW < KK;
   bool res = false;
@@ -378,8 +386,8 @@ __global__ __launch_bounds__(kThr, 2) void prefill(PreArgs A, KVLayers kv) {
           const int c = 32 * (kk >> 1) + 8 * (jj & 3) + 2 * (2 * (kk & 1) + h) + (jj >> 2);
           a2[y] = A.alpha * A.signs[c];
           const float hf = static_cast<float>(static_cast<_Float16>(a2[y]));
-          e2[y] = a2[y] - hf;
-          res |= fabsf(e2[y]) > 4e-5f * fabsf(a2[y]);
+          e2[y] = a2[y] - fmaf(hf, A.ae, hf);
+          res |= fabsf(e2[y]) > 1e-6f * fabsf(a2[y]);
           a2[y] = -hf;
         }
         s4[j] = pk(a2[0], a2[1]);
@@ -534,19 +542,27 @@ __global__ __launch_bounds__(kThr, 2) void prefill(PreArgs A, KVLayers kv) {
 
       // scores: rows tokens, this lane's column its query row
       v16f S = {};
-#pragma unroll
-      for (int kk = 0; kk < KK; ++kk) {
-        const uint8_t* at = buf + kk * 1024 + lane * 16;
-        const v4u ka = *reinterpret_cast<const v4u*>(at);
-        const v4u sa = *reinterpret_cast<const v4u*>(at + C::OFF_S);
+      auto qjl = [&](int kk) {
+        const v4u sa = *reinterpret_cast<const v4u*>(buf + kk * 1024 + lane * 16 + C::OFF_S);
         // (opaque: as loop invariants wh and wl would take 64 registers and spill)
         asm volatile("" : "+v"(qhi[kk]));
         // |q~| = |hi| + lo sign(hi)
         const v4u wh = qhi[kk] & 0x7fff7fffu, wl = qlo[kk] ^ (qhi[kk] & 0x80008000u);
-        S = mfma_h(ka, qhi[kk], S);
         S = mfma_h(sa, wh, S);
-        S = mfma_h(ka, qlo[kk], S);
         S = mfma_h(sa, wl, S);
+      };
+      if constexpr (C::AE) {  // the whole QJL term first, to mend its weight
+#pragma unroll
+        for (int kk = 0; kk < KK; ++kk) qjl(kk);
+        S *= 1.f + A.ae;
+      }
+#pragma unroll
+      for (int kk = 0; kk < KK; ++kk) {
+        const uint8_t* at = buf + kk * 1024 + lane * 16;
+        const v4u ka = *reinterpret_cast<const v4u*>(at);
+        S = mfma_h(ka, qhi[kk], S);
+        if constexpr (!C::AE) qjl(kk);
+        S = mfma_h(ka, qlo[kk], S);
         if constexpr (C::KLO)
           S = mfma_h(*reinterpret_cast<const v4u*>(at + C::SEG), qhi[kk], S);
       }
@@ -817,7 +833,7 @@ void fill_levels(const float* cent, int bits, float s, Levels* lv) {
 struct PreLevels {
   Levels kl, vl;
   float ks;
-  bool fits;  // levels and QJL weight well inside f16's range at their scales
+  bool fits;  // levels and QJL weight inside f16's range at their scales, single levels exact
 };
 
 // Largest positive magnitude of a symmetric codebook (its upper half, in any order).
@@ -848,10 +864,9 @@ const PreLevels& levels_for(int d, int kbits, int vbits, const float* kc, const 
   memcpy(m.kc, kc, nk);
   memcpy(m.vc, vc, nv);
   const float* kp = kc + (1 << (kbits - 1));
-  const float* vp = vc + (1 << (vbits - 1));
   // where the key levels keep hi + lo, their scale serves the QJL weight alone
   if (!key_lo(d, kbits)) {
-    m.lv.ks = best_scale(kp, 1 << (kbits - 1), fabsf(alpha), 0.1f);
+    m.lv.ks = best_scale(kp, 1 << (kbits - 1), fabsf(alpha), 0.003f);
   } else {
     const float top = top_level(kc, kbits);
     const float lo = alpha != 0.f ? fabsf(alpha) : top;
@@ -862,11 +877,13 @@ const PreLevels& levels_for(int d, int kbits, int vbits, const float* kc, const 
     const float ma = frexpf(lo, &ea);
     m.lv.ks = ldexpf(1.f / ma, 4 - e);
   }
-  const float vs = vbits <= 2 ? best_scale(vp, 1 << (vbits - 1), 0.f, 0.f)
-                              : 16.f / top_level(vc, vbits);
+  const float vs = 16.f / top_level(vc, vbits);
   auto in_f16 = [](float x) { return x <= 32768.f; };  // (false for NaN)
   m.lv.fits = m.lv.ks > 0.f && vs > 0.f && in_f16(top_level(kc, kbits) * m.lv.ks) &&
               in_f16(fabsf(alpha) * m.lv.ks) && in_f16(top_level(vc, vbits) * vs);
+  if (!key_lo(d, kbits))  // (a rare pair of magnitudes has no such scale)
+    for (int c = 0; c < 1 << (kbits - 1); ++c)
+      m.lv.fits &= fabsf(f16_round(kp[c] * m.lv.ks) - kp[c] * m.lv.ks) <= 2e-6f * kp[c] * m.lv.ks;
   fill_levels(kc, kbits, m.lv.ks, &m.lv.kl);
   fill_levels(vc, vbits, vs, &m.lv.vl);
   return m.lv;
@@ -935,6 +952,8 @@ int qkv_prefill(const QkvPrefillArgs& a, hipStream_t s) {
   A.pi = a.pi;
   A.signs = a.signs;
   A.alpha = a.qjl_scale * lv.ks;
+  const float ah = f16_round(A.alpha);
+  if (a.kbits == 2 && !key_lo(a.d, 2) && ah != 0.f) A.ae = A.alpha / ah - 1.f;
   A.c0 = a.scale * 1.4426950408889634f / lv.ks;
   A.causal = a.causal;
   A.split_len = ((a.T + a.n_splits - 1) / a.n_splits + 63) / 64 * 64;

@@ -161,9 +161,8 @@ def test_prefill_large_logits_and_norms(kb, vb):
     ref, top = exact(e, q, True, logits=True)
     out = e.attention(q, causal=True)
     err = (out.double() - ref).norm(dim=-1) / ref.norm(dim=-1).clamp(min=1e-30)
-    # a score is good to 4e-6 of itself (the f16 key levels: 1e-6, and 2.5e-5 of the
-    # QJL term, a ninth of it), so a row moves by at most that of the largest logit;
-    # the decode kernels' error here is 3e-2 on average
+    # a score good to 4e-6 of itself moves a row by at most that of the largest logit
+    # (key levels are good to 5e-7); the decode kernels' error here is 3e-2 on average
     assert float(err.max()) <= 4e-6 * top + 2e-5 and float(err.mean()) <= 2e-5
 
 
@@ -311,3 +310,16 @@ def test_prefill_non_finite_norms_behind_the_mask(d, splits):
         i = slot - (T - Q)   # the first query that sees it
         check(out[:, :, :i], ref[:, :, :i])
         assert not torch.isfinite(out[:, :, i:]).all(-1).any()
+
+
+@pytest.mark.parametrize("d,kb,vb,scale,bar", [
+    # logits up to ~130: the QJL weight in one f16 (2.5e-5 off) gave 1.5e-5
+    (128, 3, 3, 8.0, 3e-6), (96, 3, 3, 8.0, 3e-6),
+    # logits near 0: two value magnitudes in one f16 each gave 4.5e-7 - 6e-7; the
+    # rounding of ~150 fp32 additions per output, 2^-24 sqrt(150 / 12), is 2e-7
+    (64, 2, 2, 0.05, 3.5e-7), (96, 3, 2, 0.05, 3.5e-7), (128, 3, 2, 0.05, 3.5e-7),
+])
+def test_prefill_precision(d, kb, vb, scale, bar):
+    e, g = filled(4, 8, 777, d, kb, vb, 29, dtype=torch.float32)
+    q = scale * torch.randn(4, 32, 64, d, device=DEV, generator=g)
+    check(e.attention(q, causal=True), exact(e, q, True), bar)
