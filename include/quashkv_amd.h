@@ -302,6 +302,8 @@ int qkv_vtiles_unpack(const uint32_t* src, int64_t groups, int64_t S, int32_t d,
  *   t_stride   token capacity (multiple of 32; 64 for the MFMA path)
  *   T          valid tokens (<= t_stride); causal masks kv_pos > T - Q + i
  *   kcent_host, vcent_host  HOST arrays of the 2^kbits / 2^vbits centroids
+ *   signs      d fp32, the QJL sign vector S: +-1 (other magnitudes within
+ *              1e-3 .. 1e3 of each other and of 1 are served as they are)
  *   out        B x Hq x Q x d, out_dtype
  *   workspace  >= qkv_attention_workspace_bytes(..., n_splits), 256-B aligned
  * Symmetric codebooks (all Lloyd-Max codebooks are) with d = 128 and

@@ -496,11 +496,15 @@ __global__ __launch_bounds__(kThr, 2) void prefill(PreArgs A, KVLayers kv) {
       if (h == 0) {
         // a value norm that is not finite: weight 0 times 0 where the slot is masked, a
         // reference of infinity (NaN out) for the rows that see it
-        const bool fin = wave == 0 || fabsf(r.nm) < INFINITY;
-        nm[32 * wave + n] = wave == 0 ? r.nm * A.c0 : fin ? r.nm : 0.f;
+        float nv = wave == 0 ? r.nm * A.c0 : r.nm;
         // log2, from 2^-90 up: a row of zero norms alone keeps finite weights
-        if (wave == 1)
-          nm[64 + n] = fin ? __builtin_amdgcn_logf(fmaxf(fabsf(r.nm), kMinNorm)) : INFINITY;
+        float lg = __builtin_amdgcn_logf(fmaxf(fabsf(nv), kMinNorm));
+        if (__builtin_expect(wave == 1 && !(fabsf(nv) < INFINITY), 0)) {
+          nv = 0.f;
+          lg = INFINITY;
+        }
+        nm[32 * wave + n] = nv;
+        if (wave == 1) nm[64 + n] = lg;
       }
     }
   };
