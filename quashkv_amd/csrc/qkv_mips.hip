@@ -1085,7 +1085,7 @@ MipsPlan mips_plan(int32_t M, int64_t N, int k) {
 // need a byte value past 64 (the full scan then runs).
 bool filt_table(const float* kc, int mbits, float qjl_scale, FiltTab* ft) {
   const int n = 1 << mbits;
-  const float cmax = kc[n - 1];
+  const float cmax = *std::max_element(kc, kc + n);  // (a caller's codebook may be in any order)
   bool found = false;
   for (int lm = 8; lm <= 100; ++lm) {
     const float a = cmax / lm;

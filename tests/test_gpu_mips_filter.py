@@ -86,3 +86,13 @@ def test_sorted_database_and_batches():
     idx = QuashIndex(dim=d, bits=3, seed=3, device=DEV)
     idx.add(db)
     _same(idx, q, 10)
+
+
+@pytest.mark.parametrize("bits,cent", [(3, (-1, -20, 20, 1)), (4, (-1, -40, -30, -2, 2, 30, 40, 1))])
+def test_codebooks_in_any_order(bits, cent):
+    g = torch.Generator(device=DEV).manual_seed(7)
+    idx = QuashIndex(dim=128, bits=bits, seed=3, device=DEV)
+    idx.add(torch.randn(30000, 128, device=DEV, generator=g))
+    own = idx._host_tables()
+    idx._host_tables = lambda: (N.HostFloats([0.03 * c for c in cent]), *own[1:])
+    _same(idx, torch.randn(40, 128, device=DEV, generator=g), 10)
