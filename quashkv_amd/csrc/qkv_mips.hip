@@ -492,9 +492,11 @@ __global__ __launch_bounds__(256) void mips_fprep(const float* __restrict__ qw,
     const float slack = 1.9e-6f * (2.f * ft.a * ft.lmax * l1 + 4.f * aw + fabsf(cr)) +
                         65536.f * rowc[int64_t(qc) * 2 + 1];
     const float e = er * ft.lmax + ft.delta * l1 + slack;
-    const bool use = ok && fabsf(cr) < 1e30f;
-    ciu[q] = use ? static_cast<int>(ceilf((e + vq * eu - sw) * rf)) + 1 : 0;
-    cil[q] = use ? static_cast<int>(floorf((-e - vq * el - sw) * rf)) - 1 : 0;
+    const float up = (e + vq * eu - sw) * rf, low = (-e - vq * el - sw) * rf;
+    // (bounds that int32 sums hold; QJL weights far past the digits give larger ones)
+    const bool use = ok && fabsf(cr) < 1e30f && fabsf(up) < 1e9f && fabsf(low) < 1e9f;
+    ciu[q] = use ? static_cast<int>(ceilf(up)) + 1 : 0;
+    cil[q] = use ? static_cast<int>(floorf(low)) - 1 : 0;
     cnt[q] = use || q >= M ? 0 : cap + 1;  // past cap: left to the full scan
   }
   __syncthreads();

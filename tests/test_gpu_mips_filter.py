@@ -96,3 +96,13 @@ def test_codebooks_in_any_order(bits, cent):
     own = idx._host_tables()
     idx._host_tables = lambda: (N.HostFloats([0.03 * c for c in cent]), *own[1:])
     _same(idx, torch.randn(40, 128, device=DEV, generator=g), 10)
+
+
+@pytest.mark.parametrize("size", [1e4, 1e6, 1e9])
+def test_large_signs(size):
+    """QJL weights whose bounds are past int32 in units of a digit."""
+    g = torch.Generator(device=DEV).manual_seed(8)
+    idx = QuashIndex(dim=128, bits=3, seed=3, device=DEV)
+    idx.add(torch.randn(30000, 128, device=DEV, generator=g))
+    idx.quantizer.S = idx.quantizer.S * size
+    _same(idx, torch.randn(40, 128, device=DEV, generator=g), 10)
