@@ -328,6 +328,16 @@ int32_t qkv_attention_path(int32_t d, int32_t kbits, int32_t vbits,
                            const float* kcent_host, const float* vcent_host,
                            int64_t t_stride, int64_t T, int32_t n_splits);
 
+/* Splits that the prefill kernel (128 query rows per workgroup) runs for a
+ * single call with these parameters, 0 where the decode kernels are the faster
+ * ones or it does not take the codebooks, -1 for invalid arguments.  ranges: the
+ * call has kv_start, kv_end or q_end. */
+int32_t qkv_attention_prefills(int32_t B, int32_t Hq, int32_t Hkv, int32_t Q,
+                               int32_t d, int64_t T, int32_t kbits, int32_t vbits,
+                               const float* kcent_host, const float* vcent_host,
+                               float qjl_scale, int64_t t_stride, int32_t ranges,
+                               int64_t ws_bytes, int32_t n_splits);
+
 int qkv_decode_attention(const void* q, int32_t q_dtype, const uint8_t* kstore,
                          const float* knorm, const uint32_t* vstore,
                          const float* vnorm, int64_t t_stride, int64_t T,

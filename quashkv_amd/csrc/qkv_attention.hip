@@ -2245,18 +2245,23 @@ static int32_t decode_splits(int32_t B, int32_t Hq, int32_t Hkv, int32_t Q, int3
 // Whether the prefill kernel is the faster one for R query rows in each of bh
 // (sequence, kv head) groups over T keys, ds splits of the decode kernels against
 // ps of its own: both kernels' times in us as measured (rounds of the chip's
-// workgroups times their steps; fixed part; the merge of splits).  E.g. d = 128, 8 groups: 48 rows over 256 keys 19 against 28 us, over
-// 8192 keys 51 against 37; 256 rows over 2048 keys 42 against 39; 8192 rows over
-// 2048 keys 1052 against 144.
-static bool prefill_pays(int64_t bh, int R, int32_t d, int64_t T, int ds, int ps) {
+// workgroups times their steps; fixed part; the merge of splits).  E.g. d = 128, 8
+// groups: 48 rows over 256 keys 19 against 28 us, over 8192 keys 51 against 37; 256
+// rows over 2048 keys 42 against 39; 8192 rows over 2048 keys 1052 against 155.
+// small: decode_small serves the call (d = 64, key MSE bits <= 2, no key ranges); at
+// d = 64 decode_fused is a good deal slower (96 groups of 287 rows over 95 keys: 56 us
+// in decode_small, 301 in decode_fused with 2 key MSE bits, 413 with 3; 27 here).
+static bool prefill_pays(int64_t bh, int R, int32_t d, int64_t T, int kbits, bool small, int ds,
+                         int ps) {
   const int64_t ncu = qkv_num_cus();
   auto rounds = [&](int64_t wgs) { return static_cast<double>((wgs + ncu - 1) / ncu); };
   double dec;
-  if (d == 64) {  // decode_small: 8 rows per workgroup, three workgroups per CU
+  if (small) {  // 8 rows per workgroup, three workgroups per CU
     dec = 12.0 + 2.7e-5 * double(bh * ((R + 7) / 8)) * double(T);
-  } else {        // decode_fused: 4 rows, 512-token chunks of 2.31 us
-    dec = rounds(bh * ((R + kRowsM - 1) / kRowsM) * ds) *
-          (11.0 + 2.31 / 512.0 * double(T) / ds);
+  } else {      // decode_fused: 4 rows, a fixed part and 512-token chunks
+    const double fix = d == 64 ? (kbits == 3 ? 14.5 : 10.5) : 11.0;
+    const double chunk = d == 64 ? (kbits == 3 ? 3.3 : 1.95) : 2.31;
+    dec = rounds(bh * ((R + kRowsM - 1) / kRowsM) * ds) * (fix + chunk / 512.0 * double(T) / ds);
   }
   dec += ds > 1 ? 5.0 : 0.0;
   const double step = d == 128 ? 4.4 : d == 96 ? 3.2 : 2.0;  // per 64 tokens
@@ -2283,14 +2288,16 @@ static int64_t split_bytes(int64_t bh, int R, int d) { return bh * R * (int64_t(
 // 0: the call stays on the decode kernels.
 static int prefill_count(int32_t B, int32_t Hq, int32_t Hkv, int32_t Q, int32_t d, int64_t T,
                          int32_t kbits, int32_t vbits, const float* kcent, const float* vcent,
-                         float qjl_scale, int64_t t_stride, int64_t ws_bytes, int n_splits) {
+                         float qjl_scale, int64_t t_stride, bool ranges, int64_t ws_bytes,
+                         int n_splits) {
   const int R = (Hq / Hkv) * Q;
   if (R < kPrefillMinRows || t_stride % 64 != 0) return 0;
+  const bool small = d == 64 && kbits <= 2 && !ranges;
   const int64_t bh = int64_t(B) * Hkv;
   const int ds = decode_splits(B, Hq, Hkv, Q, d, T);
   const int own = static_cast<int>(std::max<int64_t>(
       1, std::min<int64_t>(qkv_prefill_splits(bh, R, d, T), ws_bytes / split_bytes(bh, R, d))));
-  if (!prefill_pays(bh, R, d, T, ds, own) ||
+  if (!prefill_pays(bh, R, d, T, kbits, small, ds, own) ||
       !qkv_prefill_ok(d, kbits, vbits, kcent, vcent, qjl_scale))
     return 0;
   return n_splits == ds ? own : n_splits;
@@ -2327,6 +2334,18 @@ extern "C" int64_t qkv_attention_workspace_bytes(int32_t B, int32_t Hq, int32_t 
   if (R < kPrefillMinRows || !qkv_d_ok(d)) return need;
   const int64_t bh = int64_t(B) * Hkv;
   return std::max(need, qkv_prefill_splits(bh, R, d, INT64_MAX) * split_bytes(bh, R, d));
+}
+
+extern "C" int32_t qkv_attention_prefills(int32_t B, int32_t Hq, int32_t Hkv, int32_t Q,
+                                          int32_t d, int64_t T, int32_t kbits, int32_t vbits,
+                                          const float* kcent_host, const float* vcent_host,
+                                          float qjl_scale, int64_t t_stride, int32_t ranges,
+                                          int64_t ws_bytes, int32_t n_splits) {
+  if (B <= 0 || Hkv <= 0 || Hq <= 0 || Q <= 0 || Hq % Hkv != 0 || T <= 0 || n_splits < 1 ||
+      !qkv_d_ok(d) || !qkv_bits_ok(kbits) || !qkv_bits_ok(vbits) || !kcent_host || !vcent_host)
+    return -1;
+  return prefill_count(B, Hq, Hkv, Q, d, T, kbits, vbits, kcent_host, vcent_host, qjl_scale,
+                       t_stride, ranges != 0, ws_bytes, n_splits);
 }
 
 extern "C" int32_t qkv_attention_path(int32_t d, int32_t kbits, int32_t vbits,
@@ -2640,14 +2659,15 @@ int decode_attention_impl(const void* q, int32_t q_dtype, const uint8_t* kstore,
   kv.khi = kr.khi;
   kv.cbase = kr.cbase;
   auto s = static_cast<hipStream_t>(stream);
+  const bool ranges = kr.klo || kr.khi || kr.cbase != 0;
   const int ps = prefill_count(B, Hq, Hkv, Q, d, T, kbits, vbits, kcent_host, vcent_host,
-                               qjl_scale, t_stride, ws_bytes, n_splits);
+                               qjl_scale, t_stride, ranges, ws_bytes, n_splits);
   if (ps > 0)
     return run_prefill(q, q_dtype, kv, t_stride, T, B, Hq, Hkv, Q, d, kbits, vbits, pi,
                        kcent_host, vcent_host, signs, qjl_scale, scale, causal, out, out_dtype,
                        workspace, ps, s);
   const Tables tb = make_tables(kcent_host, kbits, vcent_host, vbits);
-  if (d == 64 && tb.mfma_ok && t_stride % 64 == 0 && !kr.klo && !kr.khi && kr.cbase == 0) {
+  if (d == 64 && tb.mfma_ok && t_stride % 64 == 0 && !ranges) {
     // decode_small: one launch (plus combine_kernel with several splits)
     QKV_REQUIRE(qkv_aligned(pi, 16) && qkv_aligned(kstore, 4) && qkv_aligned(vstore, 4),
                 "pi must be 16-byte and the store 4-byte aligned");
@@ -2839,7 +2859,7 @@ extern "C" int qkv_paged_decode_attention(
   kv.plg = plg;
   kv.npages = num_pages;
   const int ps = prefill_count(B, Hq, Hkv, Q, d, T, kbits, vbits, kcent_host, vcent_host,
-                               qjl_scale, t_stride, ws_bytes, n_splits);
+                               qjl_scale, t_stride, false, ws_bytes, n_splits);
   if (ps > 0)
     return run_prefill(q, q_dtype, kv, t_stride, T, B, Hq, Hkv, Q, d, kbits, vbits, pi,
                        kcent_host, vcent_host, signs, qjl_scale, scale, causal, out, out_dtype,

@@ -38,3 +38,22 @@ def test_splits_of_many_rows_serve_the_three_call_form(B, Hq, Hkv, Q, d, T, spli
     own = min(64, 256 // (B * Hkv * ((R + 127) // 128)))
     room = max(1, own) * rows * (4 * d + 8)
     assert L.qkv_attention_workspace_bytes(B, Hq, Hkv, Q, d, s) == max(layout, room)
+
+
+@pytest.mark.parametrize("B,H,R,T,kb,ranges,prefills", [
+    # decode_small serves the call: 21 us against 26
+    (20, 5, 287, 95, 3, 0, False), (20, 5, 287, 500, 3, 0, True), (1, 8, 48, 256, 3, 0, False),
+    # it does not (3 key MSE bits; key ranges): 330 and 290 us
+    (20, 5, 287, 95, 4, 0, True), (20, 5, 287, 95, 3, 1, True), (4, 8, 64, 400, 4, 0, True),
+    (1, 8, 48, 256, 4, 0, False), (1, 8, 47, 4096, 4, 0, False),
+])
+def test_prefill_rule_at_64(B, H, R, T, kb, ranges, prefills):
+    L = N.lib()
+    m = [0.05, 0.15, 0.25, 0.35][: 1 << (kb - 2)]
+    kc = N.HostFloats([-x for x in m[::-1]] + m)
+    vc = N.HostFloats([-2.0, -1.3, -0.7, -0.2, 0.2, 0.7, 1.3, 2.0])
+    s = L.qkv_attention_splits(B, H, H, R, 64, T)
+    ws = L.qkv_attention_workspace_bytes(B, H, H, R, 64, s)
+    n = L.qkv_attention_prefills(B, H, H, R, 64, T, kb - 1, 3, kc.ptr, vc.ptr, 0.02,
+                                 -(-T // 64) * 64, ranges, ws, s)
+    assert (n > 0) == prefills
