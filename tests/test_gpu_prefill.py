@@ -4,7 +4,8 @@ width, query and output dtype, GQA group, remainders of the 128-row and 32-token
 tiles, causal and full, key ranges, splits, paged stores, large logits.
 
 The shapes have enough (sequence, kv head) groups that the dispatch's cost rule
-sends them to the prefill kernel (smaller calls stay on the decode kernels).
+sends them to the prefill kernel (smaller calls stay on the decode kernels), which
+each test asserts.
 
 Bar for fp32 outputs: 3e-5 relative (2-norm), the decode kernels' own (their
 large-logit bar is 1e-4, measured 2.2e-5)."""
@@ -70,6 +71,22 @@ def exact(e, q, causal, lo=None, hi=None, q_end=0, signs=None, logits=False, kce
     return (out, top) if logits else out
 
 
+def prefills(e, q, ranges=False, n_splits=None, kcent=None, vcent=None, qjl=None):
+    """Whether the prefill kernel takes the call."""
+    L, kq, vq = N.lib(), e.key_quantizer, e.value_quantizer
+    B, Hq, Q, d = q.shape
+    H, T, cap = e._store.H, e.total_tokens, e._store.capacity
+    ns = L.qkv_attention_splits(B, Hq, H, Q, d, T)
+    kc = N.HostFloats(kcent or kq.mse_quantizer.codebook.centroids_host)
+    vc = N.HostFloats(vcent or vq.codebook.centroids_host)
+    n = L.qkv_attention_prefills(B, Hq, H, Q, d, T, kq.mse_bits, vq.bits, kc.ptr, vc.ptr,
+                                 kq.qjl_scale if qjl is None else qjl, cap, ranges,
+                                 L.qkv_attention_workspace_bytes(B, Hq, H, Q, d, n_splits or ns),
+                                 n_splits or ns)
+    assert n >= 0
+    return n > 0
+
+
 def check(out, ref, bar=3e-5):
     err = float((out.double() - ref).norm() / ref.norm())
     assert err <= bar, err
@@ -89,12 +106,14 @@ def filled(B, H, T, d, kb, vb, seed, dtype=torch.bfloat16, cls=quashkv.QuashKVEn
 @pytest.mark.parametrize("kb,vb", [(2, 1), (2, 2), (3, 3), (3, 4), (4, 4), (4, 2)])
 @pytest.mark.parametrize("B,G,H,T,Q,causal,dtype", [
     (8, 4, 8, 160, 33, True, torch.bfloat16),   # 132 rows: a 4-row remainder
-    (20, 7, 5, 95, 41, False, torch.float16),
+    (20, 7, 5, 95, 41, False, torch.float16),   # (d = 64, 2 key MSE bits: decode_small's)
+    (20, 7, 5, 500, 41, False, torch.float16),
     (11, 1, 9, 300, 129, True, torch.float32),
 ])
 def test_prefill_matches_64_bits(d, kb, vb, B, G, H, T, Q, causal, dtype):
     e, g = filled(B, H, T, d, kb, vb, T + Q)
     q = torch.randn(B, H * G, Q, d, device=DEV, generator=g).to(dtype)
+    assert prefills(e, q) == (d != 64 or kb > 3 or T != 95)
     ref = exact(e, q, causal)
     check(e.attention(q, causal=causal), ref)
     check(e.attention(q, causal=causal, out_dtype=torch.bfloat16).float(), ref, 4e-3)
@@ -107,6 +126,7 @@ def test_prefill_sizes(T, Q, G):
     """The smallest calls, whole and odd numbers of tiles, Q = T."""
     e, g = filled(8, 8, T, 128, 3, 3, T)
     q = torch.randn(8, 8 * G, Q, 128, device=DEV, generator=g)
+    assert prefills(e, q)
     check(e.attention(q, causal=True), exact(e, q, True))
 
 
@@ -114,6 +134,7 @@ def test_prefill_sizes(T, Q, G):
 def test_prefill_splits(d, splits):
     e, g = filled(8, 8, 700, d, 3, 3, splits)
     q = torch.randn(8, 32, 60, d, device=DEV, generator=g)
+    assert prefills(e, q, n_splits=splits)
     kq, vq = e.key_quantizer, e.value_quantizer
     for causal in (False, True):
         out = attention_store(q, e._store, 700, kq.mse_quantizer.Pi,
@@ -128,6 +149,7 @@ def test_prefill_ranges_and_positions():
     q = torch.randn(4, 64, 40, 128, device=DEV, generator=g)
     lo = torch.tensor([0, 31, 32, 200], device=DEV, dtype=torch.int32)
     hi = torch.tensor([333, 300, 97, 200], device=DEV, dtype=torch.int32)   # the last: no keys
+    assert prefills(e, q, ranges=True)
     for causal, q_end in ((False, 0), (True, 0), (True, 333), (True, 60)):
         out = e.attention(q, causal=causal, kv_start=lo, kv_end=hi, q_end=q_end)
         check(out, exact(e, q, causal, lo, hi, q_end))
@@ -140,6 +162,7 @@ def test_prefill_paged_equals_contiguous(d, kb, page):
     a, g = filled(*args)
     b, _ = filled(*args, cls=PagedQuashKVEngine, page_tokens=page)
     q = torch.randn(8, 32, 60, d, device=DEV, generator=g)
+    assert prefills(a, q)
     assert torch.equal(a.attention(q, causal=True), b.attention(q, causal=True))
 
 
@@ -158,6 +181,7 @@ def test_prefill_large_logits_and_norms(kb, vb):
     q[:, :, 1] *= 1e-6
     q[:, :, 2, 1:] = 0.0
     q[:, :, 3] = 0.0
+    assert prefills(e, q)
     ref, top = exact(e, q, True, logits=True)
     out = e.attention(q, causal=True)
     err = (out.double() - ref).norm(dim=-1) / ref.norm(dim=-1).clamp(min=1e-30)
@@ -173,6 +197,7 @@ def test_prefill_other_signs():
     kq, vq = e.key_quantizer, e.value_quantizer
     signs = kq.S * (0.5 + torch.rand(128, device=DEV, generator=g))
     signs[5] = 0.0
+    assert prefills(e, q)
     out = attention_store(q, e._store, 200, kq.mse_quantizer.Pi,
                           kq.mse_quantizer.codebook.centroids_host, vq.codebook.centroids_host,
                           signs, kq.qjl_scale, causal=True)
@@ -190,6 +215,7 @@ def test_prefill_extremes(d, T):
     q[:, :, 45] *= 1e-39
     lo = torch.full((8,), 5, device=DEV, dtype=torch.int32)
     hi = torch.full((8,), T - 13, device=DEV, dtype=torch.int32)
+    assert prefills(e, q, ranges=True)
     refs = [exact(e, q, True, lo, hi, end) for end in (0, 80)]
     assert float(refs[1][:, :, :40].abs().max()) == 0.0
     st.vnorm.view(8, 8, -1)[:, :, :5] = math.inf
@@ -210,6 +236,7 @@ def test_prefill_split_large_value_norms(d, splits):
     q = torch.randn(8, 32, 60, d, device=DEV, generator=g)
     kq, vq = e.key_quantizer, e.value_quantizer
     e._store.vnorm *= torch.tensor([1e12, 1e-12] * 4, device=DEV)[:, None]
+    assert prefills(e, q, n_splits=splits)
     ref = exact(e, q, True)
     out = attention_store(q, e._store, 700, kq.mse_quantizer.Pi,
                           kq.mse_quantizer.codebook.centroids_host,
@@ -253,13 +280,14 @@ def _call(e, q, causal, form):
 
 
 @pytest.mark.parametrize("B,H,G,Q,d,T", [(8, 8, 4, 64, 64, 8192), (1, 8, 1, 128, 128, 8200),
-                                         (2, 4, 2, 64, 96, 4096)])
+                                         (2, 4, 2, 300, 96, 4096)])
 def test_many_rows_by_every_form(B, H, G, Q, d, T):
     """The split count of the library in the single call (the prefill kernel's own
     splits, also where the no-allocation array holds fewer than it asks for) and in
     the three-call form, whose kernels it is for."""
     e, g = filled(B, H, T, d, 3, 3, 17)
     q = torch.randn(B, H * G, Q, d, device=DEV, generator=g)
+    assert prefills(e, q)
     ref = exact(e, q, True)
     a = _call(e, q, True, "workspace")
     check(a, ref)
@@ -271,7 +299,7 @@ def test_many_rows_by_every_form(B, H, G, Q, d, T):
 
 @pytest.mark.parametrize("kb,vb,kc,vc,qjl", [
     (3, 2, (0.0011, 0.1), None, 95.0),            # a QJL weight past f16 at the levels' scale
-    (3, 2, None, (1.0, 2e5), None),               # value levels likewise
+    (3, 2, None, (1.0, 2e5), None),               # value levels of such a ratio
     (3, 3, (0.15, 0.05), (3e5, 0.9, 0.3, 1.0), None),   # levels in no order
     (4, 4, (0.05, 0.2, 0.1, 0.15), (.4, .1, .3, .2, .8, .5, .7, .6), None),
 ])
@@ -285,6 +313,7 @@ def test_prefill_other_codebooks(kb, vb, kc, vc, qjl):
     kc = both(kc, kq.mse_quantizer.codebook.centroids_host)
     vc = both(vc, vq.codebook.centroids_host)
     qjl = kq.qjl_scale if qjl is None else qjl
+    assert prefills(e, q, kcent=kc, vcent=vc, qjl=qjl) == (qjl < 90.0)
     out = attention_store(q, e._store, 333, kq.mse_quantizer.Pi, kc, vc, kq.S, qjl, causal=True)
     check(out, exact(e, q, True, kcent=kc, vcent=vc, qjl=qjl))
 
@@ -297,6 +326,7 @@ def test_prefill_non_finite_norms_behind_the_mask(d, splits):
     e, g = filled(8, 8, T, d, 3, 3, 23)
     q = torch.randn(8, 32, Q, d, device=DEV, generator=g)
     kq, vq = e.key_quantizer, e.value_quantizer
+    assert prefills(e, q, n_splits=splits)
     ref = exact(e, q, True)
     for slot, bad in ((T - 20, math.inf), (T - 33, math.nan)):
         norm = e._store.vnorm if bad == math.inf else e._store.knorm
@@ -322,4 +352,5 @@ def test_prefill_non_finite_norms_behind_the_mask(d, splits):
 def test_prefill_precision(d, kb, vb, scale, bar):
     e, g = filled(4, 8, 777, d, kb, vb, 29, dtype=torch.float32)
     q = scale * torch.randn(4, 32, 64, d, device=DEV, generator=g)
+    assert prefills(e, q)
     check(e.attention(q, causal=True), exact(e, q, True), bar)
