@@ -64,7 +64,7 @@ __global__ __launch_bounds__(256, 2) void mips_scan(const qkv_v4i* __restrict__ 
                                                  float* __restrict__ cand_s,
                                                  int* __restrict__ cand_i,
                                                  uint32_t* __restrict__ gth,
-                                                 const int* __restrict__ over, int cap) {
+                                                 const int* __restrict__ left) {
   using C = MipsCfg<MB, PDW>;
   constexpr int NU = C::NU, QC = C::QC, RAWD = C::RAWD;
   constexpr int QW = 4 * QC;                      // queries per wave
@@ -116,13 +116,22 @@ __global__ __launch_bounds__(256, 2) void mips_scan(const qkv_v4i* __restrict__ 
   // items (query tile, vector chunk), vector-chunk major, so that a query's
   // later chunks start from the k-th best score its earlier chunks published
   // (gth); a workgroup takes items blockIdx.x, blockIdx.x + gridDim.x, ...
-  const int qtiles = static_cast<int>(n_items / nvc);
+  // Behind the filter (left): only the query chunks it left, left[0] of them in
+  // left[1 ..].
+  int qtiles = static_cast<int>(n_items / nvc), nch = nchunks;
+  if (left != nullptr) {
+    nch = left[0];
+    qtiles = (nch + 4 * QC - 1) / (4 * QC);
+    n_items = int64_t(qtiles) * nvc;
+  }
   for (int64_t item = blockIdx.x; item < n_items; item += gridDim.x) {
     const int vc = static_cast<int>(item / qtiles), qt = static_cast<int>(item % qtiles);
-    const int chunk0 = (qt * 4 + wave) * QC;  // first query chunk of this wave
-    if (over != nullptr) {  // behind the filter: only tiles with an overflowed query
-      const int qo = qt * 4 * QW + tid;
-      if (!__syncthreads_or(tid < 4 * QW && qo < M && over[qo] > cap)) continue;
+    // this wave's query chunks (nchunks: none)
+    int chs[QC];
+#pragma unroll
+    for (int c = 0; c < QC; ++c) {
+      const int i = (qt * 4 + __builtin_amdgcn_readfirstlane(wave)) * QC + c;
+      chs[c] = i >= nch ? nchunks : left != nullptr ? left[1 + i] : i;
     }
     const int64_t v0 = int64_t(vc) * vlen;
     const int64_t v1 = min<int64_t>(N, v0 + vlen);
@@ -134,13 +143,13 @@ __global__ __launch_bounds__(256, 2) void mips_scan(const qkv_v4i* __restrict__ 
     float fq[QC], cr[QC], theta[QC], tg[QC], thr[QC];
 #pragma unroll
     for (int c = 0; c < QC; ++c) {
-      const int ch = min(chunk0 + c, nchunks - 1);
+      const int ch = min(chs[c], nchunks - 1);
 #pragma unroll
       for (int u = 0; u < NU; ++u) a[c][u] = aq[(int64_t(ch) * NU + u) * 64 + lane];
       cr[c] = rowc[(int64_t(ch) * kRowsM + lg) * 2 + 0];
       fq[c] = rowc[(int64_t(ch) * kRowsM + lg) * 2 + 1];
       theta[c] = -INFINITY;
-      const int qg = (chunk0 + c) * 4 + lg;
+      const int qg = chs[c] * 4 + lg;
       tg[c] = qg < M ? fkey_inv(__hip_atomic_load(&gth[qg], __ATOMIC_RELAXED,
                                                   __HIP_MEMORY_SCOPE_AGENT))
                      : INFINITY;
@@ -285,9 +294,13 @@ __global__ __launch_bounds__(256, 2) void mips_scan(const qkv_v4i* __restrict__ 
     }
     // this wave's lists -> candidates [query][vector chunk][k]; a full list's
     // k-th score raises the query's device-wide bound
+#pragma unroll 1
     for (int q = 0; q < QW; ++q) {
-      const int qg = (chunk0 + q / 4) * 4 + (q % 4);
-      if (qg >= M) break;
+      int ch = chs[0];
+#pragma unroll
+      for (int c = 1; c < QC; ++c) ch = q / 4 == c ? chs[c] : ch;
+      const int qg = ch * 4 + (q % 4);
+      if (qg >= M) continue;
       const int64_t base = (int64_t(qg) * nvc + vc) * k;
       for (int j = lane; j < k; j += 64) {
         cand_s[base + j] = wls[q * k + j];
@@ -363,16 +376,25 @@ __global__ __launch_bounds__(64) void mips_merge(const float* __restrict__ cand_
 //      of vectors, so mips_bound's k-th largest of them bounds the k-th best
 //      score from below;
 //   2. mips_pass<true> lists the vectors whose upper bound reaches that bound
-//      (about 25 k per query on N(0, 1) data): every vector of the exact top k,
-//      ties included, is among them;
+//      (about 25 times k per query on N(0, 1) data): every vector of the exact top
+//      k, ties included, is among them;
 //   3. mips_pick scores the listed vectors with all four digits, the same
 //      integers and float operations as the full scan, and takes the k best.
-// A query whose list overflows, or whose weights are not finite or all zero,
-// goes to the full scan.  The results are the full scan's bit for bit.
+// A query whose list overflows (or is seen in step 1 to be about to), or whose
+// weights are not finite or all zero, goes to the full scan, with its 4-query chunk;
+// the scan starts from its bound of step 1.  The results are the full scan's bit for
+// bit.
 //
-// Measured (10^6 vectors, 10^4 queries, d = 128, 3 bits, top-10): 3.02 ms against
-// the full scan's 13.1: pass 2 ~2.4 ms (matrix cores busy ~45 %; MFMA time 1.06
-// ms), pass 1 0.3, the exact scores 0.19.  QT = 4 / 6 / 8: 3.98 / 3.22 / 3.02 ms.
+// Measured (10^6 L2-normalised N(0, 1) vectors, 10^4 queries, d = 128, 3 bits,
+// top-10): 3.02 - 3.19 ms against the full scan's 13.1: pass 2 ~2.4 ms (matrix cores
+// busy ~45 %; MFMA time 1.06 ms), pass 1 0.3, the exact scores 0.19.  QT = 4 / 6 / 8:
+// 3.98 / 3.22 / 3.02 ms.  Other data, against the full scan alone: norms that differ
+// (the float products) 8.0 ms against 13.0; 1,000 clusters of spread 0.1 - 0.5 of
+// their centres' 3.2 - 3.5; 100 clusters of spread 0.05, where lists of 10,000 would
+// overflow, 12.3 against 13.0; every vector 2,000 times 12.1 against 12.4, a twentieth
+// of them so 6.1 against 13.1 (1 query over 10^5: 112 us against 119).  Without the
+// overflows foreseen and with whole 64-query tiles sent to the full scan the last
+// four were 16.8, 16.1, 16.0 ms and 163 us.
 // Six bit-plane operands in place of the level bytes (one digit, band twice as
 // wide, 24 MFMAs per 64 queries) left half of the lists past their cap.
 //
@@ -419,13 +441,18 @@ __global__ __launch_bounds__(256) void mips_fprep(const float* __restrict__ qw,
                                                   const float* __restrict__ rowc, int M,
                                                   FiltTab ft, uint32_t* __restrict__ af,
                                                   int* __restrict__ ciu, int* __restrict__ cil,
-                                                  int* __restrict__ cnt, int cap) {
+                                                  int* __restrict__ cnt, int cap,
+                                                  float* __restrict__ unit,
+                                                  int* __restrict__ left,
+                                                  int* __restrict__ claimed) {
   constexpr int NU = FiltCfg<PDW>::NU, NWD = NU * 256;
   constexpr int JT = PDW * 2;  // coordinates per thread
   __shared__ uint32_t img[NWD];
   int8_t* ib = reinterpret_cast<int8_t*>(img);
   const int tid = threadIdx.x, m = tid >> 4, t16 = tid & 15;
   for (int i = tid; i < NWD; i += 256) img[i] = 0;
+  if (tid < 4) claimed[blockIdx.x * 4 + tid] = 0;  // no chunk left to the full scan yet
+  if (blockIdx.x == 0 && tid == 0) left[0] = 0;
   const int q = blockIdx.x * 16 + m, qc = min(q, M - 1);
   float v[JT], w[JT];
   float mx = 0.f, l1 = 0.f, sw = 0.f, aw = 0.f;
@@ -498,6 +525,7 @@ __global__ __launch_bounds__(256) void mips_fprep(const float* __restrict__ qw,
     ciu[q] = use ? static_cast<int>(ceilf(up)) + 1 : 0;
     cil[q] = use ? static_cast<int>(floorf(low)) - 1 : 0;
     cnt[q] = use || q >= M ? 0 : cap + 1;  // past cap: left to the full scan
+    unit[q] = f;
   }
   __syncthreads();
   for (int i = tid; i < NWD; i += 256) af[int64_t(blockIdx.x) * NWD + i] = img[i];
@@ -520,7 +548,7 @@ template <int MB, int PDW, int QT, bool COLLECT>
 __global__ __launch_bounds__(256, 2) void mips_pass(
     const qkv_v4i* __restrict__ af, const int* __restrict__ cinit, const float* __restrict__ thr,
     const uint8_t* __restrict__ kst, const float* __restrict__ norms, int64_t N, int ntile,
-    int wq, int pb, int64_t ng, int gstep, FiltTab ft, float* __restrict__ mxo,
+    int wq, int pb, int64_t ng, int gstep, int M, FiltTab ft, float* __restrict__ mxo,
     int* __restrict__ cnt, int* __restrict__ cand, int cap) {
   constexpr int NU = FiltCfg<PDW>::NU, RAWD = (MB + 1) * PDW, NP = MB + 1;
   constexpr int NI = PDW == 2 ? 4 : 8;  // bits of each byte a lane expands
@@ -545,9 +573,38 @@ __global__ __launch_bounds__(256, 2) void mips_pass(
 #pragma unroll
     for (int u = 0; u < NU; ++u)
       a[t][u] = af[((int64_t(tile) * QT + t) * NU + u) * 64 + lane];
-  for (int i = lane; i < 16 * QT; i += 64) {
-    cis[wave][i] = cinit[int64_t(tile) * 16 * QT + i];
-    if constexpr (COLLECT) ths[wave][i] = thr[int64_t(tile) * 16 * QT + i];
+  if constexpr (!COLLECT) {
+    for (int i = lane; i < 16 * QT; i += 64) cis[wave][i] = cinit[int64_t(tile) * 16 * QT + i];
+  } else {
+    // A 4-query chunk with a query left to the full scan goes there whole (the scan
+    // takes it at the same cost), and so does a tile of whose chunks fewer than a
+    // fifth remain: this pass costs a fifth of the scan.  (Every wave of the tile
+    // decides alike, before any lists.)
+    const int q0 = tile * 16 * QT;
+    bool real = false, keep = false;
+    if (lane < 4 * QT) {
+      real = keep = q0 + 4 * lane < M;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float th = thr[q0 + 4 * lane + r];
+        if (q0 + 4 * lane + r < M && th != th) keep = false;
+      }
+    }
+    const uint64_t kept = __builtin_amdgcn_ballot_w64(keep);
+    const bool few = 5 * __builtin_popcountll(kept) <
+                     __builtin_popcountll(__builtin_amdgcn_ballot_w64(real));
+    bool some = false;
+    for (int i = lane; i < 16 * QT; i += 64) {
+      float th = thr[q0 + i];
+      if (few || !((kept >> (i / 4)) & 1u)) {
+        if (th == th) cnt[q0 + i] = cap + 1;
+        th = __builtin_nanf("");
+      }
+      cis[wave][i] = cinit[q0 + i];
+      ths[wave][i] = th;
+      some |= th == th;
+    }
+    if (__builtin_amdgcn_ballot_w64(some) == 0) return;
   }
   // COLLECT: minus the integer thresholds at nq; else the largest I at nq
   qkv_v4i ti[COLLECT ? QT : 1];
@@ -612,6 +669,7 @@ __global__ __launch_bounds__(256, 2) void mips_pass(
   };
 
   int qn = 0;  // queued candidates (wave-uniform)
+  bool done = false;  // every query's list is past its cap
   auto flush = [&]() {
     bool any = false;
     for (int i = lane; i < qn; i += 64) {
@@ -626,7 +684,12 @@ __global__ __launch_bounds__(256, 2) void mips_pass(
       }
     }
     qn = 0;
-    if (__builtin_amdgcn_ballot_w64(any)) nq = -1.f;  // (new integer thresholds)
+    if (__builtin_amdgcn_ballot_w64(any)) {
+      nq = -1.f;  // (new integer thresholds)
+      bool alive = false;
+      for (int i = lane; i < 16 * QT; i += 64) alive |= ths[wave][i] == ths[wave][i];
+      done = __builtin_amdgcn_ballot_w64(alive) == 0;
+    }
   };
 
   // COLLECT: minus the smallest I that may pass at norms in (0.999 nq, nq]
@@ -792,6 +855,7 @@ __global__ __launch_bounds__(256, 2) void mips_pass(
   for (int64_t x = p; x < ng; x += 2 * P) {
     body(b0, n0, b1, n1, r0, x);
     if (x + P < ng) body(b1, n1, b0, n0, r1, x + P);
+    if (COLLECT && done) break;
   }
   if constexpr (COLLECT) {
     flush();
@@ -810,11 +874,22 @@ __global__ __launch_bounds__(256, 2) void mips_pass(
 // Threshold of one query per workgroup: the k-th largest of 256 R maxima, each
 // the largest of a disjoint share of the query's n stream maxima, lowered by the
 // rounding of one float product.  NaN (admits nothing) for a query the filter
-// does not serve: past the cap already, or without k finite maxima.
+// does not serve: past the cap already, without k finite maxima, or with so many
+// shares whose upper bound reaches the threshold (at the mean of 64 norms) that its
+// list would overflow: v sampled vectors fall on c of S shares, v ~ -S ln(1 - c / S),
+// and step times as many are listed.  (10^6 vectors, 2,000 copies of each, 10^4
+// queries: pass 2 was 2.4 ms of 16.1, the full scan alone takes 12.4.)  In units of a
+// score the threshold is where the full scan of such a query starts from (gth),
+// instead of filling its lists (100 queries, 10^5 such vectors: 790 us, now 246; the
+// full scan alone 570).
 template <int R>
 __global__ __launch_bounds__(256) void mips_bound(const float* __restrict__ mx, int n, int k,
-                                                  int M, float* __restrict__ thr,
-                                                  int* __restrict__ cnt, int cap) {
+                                                  int M, int step, const float* __restrict__ unit,
+                                                  const int* __restrict__ ciu,
+                                                  const int* __restrict__ cil,
+                                                  const float* __restrict__ norms, int64_t N,
+                                                  float* __restrict__ thr, int* __restrict__ cnt,
+                                                  int cap, uint32_t* __restrict__ gth) {
   __shared__ float sh[256 * R];
   const int q = blockIdx.x, tid = threadIdx.x;
   if (q >= M || cnt[q] > cap) {
@@ -850,10 +925,22 @@ __global__ __launch_bounds__(256) void mips_bound(const float* __restrict__ mx, 
         }
     }
   }
+  const float t = kth - fabsf(kth) * 1.9e-6f;
+  float nm = norms[tid * (N / 64)];
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) nm += __shfl_xor(nm, o, 64);
+  const float reach = t - static_cast<float>(ciu[q] - cil[q]) * (nm * (1.f / 64.f));
+  int c = k;  // shares that reach it (the k best were taken out above)
+#pragma unroll
+  for (int x = 0; x < 4 * R; ++x) c += __builtin_popcountll(__builtin_amdgcn_ballot_w64(v[x] >= reach));
   if (tid == 0) {
     const bool ok = fabsf(kth) < INFINITY;  // else: left to the full scan
-    thr[q] = ok ? kth - fabsf(kth) * 1.9e-6f : __builtin_nanf("");
-    if (!ok) cnt[q] = cap + 1;
+    const float S = 256.f * R, est = step * S * -logf(fmaxf(1.f - c / S, 1e-6f));
+    const bool list = ok && est <= cap;
+    thr[q] = list ? t : __builtin_nanf("");
+    if (!list) cnt[q] = cap + 1;
+    const float s = t * unit[q], lo = s - fabsf(s) * 2e-6f - 1e-36f;
+    if (ok && fabsf(lo) < 1e38f) gth[q] = fkey(lo);
   }
 }
 
@@ -868,6 +955,7 @@ __global__ __launch_bounds__(256) void mips_pick(const qkv_v4i* __restrict__ aq,
                                                  const float* __restrict__ norms, int k,
                                                  const int* __restrict__ cnt,
                                                  const int* __restrict__ cand, int cap,
+                                                 int* __restrict__ left, int* __restrict__ claimed,
                                                  float* __restrict__ out_s,
                                                  int64_t* __restrict__ out_i) {
   using F = MipsCfg<MB, PDW>;
@@ -878,7 +966,10 @@ __global__ __launch_bounds__(256) void mips_pick(const qkv_v4i* __restrict__ aq,
   extern __shared__ __align__(16) float smem_mk[];  // [cap] scores, [cap] indices
   const int q = blockIdx.x, tid = threadIdx.x;
   const int n = cnt[q];
-  if (n > cap) return;
+  if (n > cap) {  // the query's chunk goes to the full scan
+    if (tid == 0 && atomicExch(&claimed[q / 4], 1) == 0) left[1 + atomicAdd(&left[0], 1)] = q / 4;
+    return;
+  }
   float* cs = smem_mk;
   int* ci = reinterpret_cast<int*>(smem_mk + cap);
   // digit v of the weight at virtual bit (plane, coordinate) from the operand image
@@ -1017,7 +1108,7 @@ namespace {
 
 struct MipsLayout {
   int64_t aq, rowc, cs, ci, gth, pad;
-  int64_t qw, af, ciu, cil, cnt, thr, mx, cand;  // the filter's
+  int64_t qw, af, ciu, cil, cnt, thr, unit, left, claimed, mx, cand;  // the filter's
   int64_t total;
 };
 
@@ -1042,7 +1133,7 @@ struct MipsPlan {
   int qt, wq, pb, P, ntile, cap, step;
 };
 
-// Listed vectors a query may have (about 25 k on N(0, 1) data), and the queries
+// Listed vectors a query may have (about 25 times k on N(0, 1) data), and the queries
 // per batch that this allows (64 MiB of lists).
 int filt_cap(int k) { return std::max(1024, 64 * k); }
 int filt_batch(int k) { return 16384 * 1024 / filt_cap(k); }
@@ -1130,6 +1221,9 @@ MipsLayout mips_layout(int32_t M, int d, int mbits, int k, int nsplit, const Mip
     w.cil = off;  off += up(mq * 4);
     w.cnt = off;  off += up(mq * 4);
     w.thr = off;  off += up(mq * 4);
+    w.unit = off; off += up(mq * 4);
+    w.left = off; off += up((1 + mq / 4) * 4);  // count, then query chunks
+    w.claimed = off; off += up(mq / 4 * 4);
     w.mx = off;   off += up(mq * 16 * pl.P * 4);
     w.cand = off; off += up(mq * pl.cap * 4);
   }
@@ -1161,8 +1255,8 @@ struct MipsArgs {
 };
 
 template <int MB, int PDW>
-int launch_scan(const MipsArgs& a, void* ws, const MipsLayout& L, int nsplit, const int* over,
-                int cap, hipStream_t s) {
+int launch_scan(const MipsArgs& a, void* ws, const MipsLayout& L, int nsplit, const int* left,
+                const int* over, int cap, hipStream_t s) {
   const int chunks = (a.M + kRowsM - 1) / kRowsM;
   constexpr int qc = MipsCfg<MB, PDW>::QC;
   const int64_t vlen = ((a.N + nsplit - 1) / nsplit + kMipsStep - 1) / kMipsStep * kMipsStep;
@@ -1183,7 +1277,7 @@ int launch_scan(const MipsArgs& a, void* ws, const MipsLayout& L, int nsplit, co
   hipLaunchKernelGGL((mips_scan<MB, PDW>), grid, dim3(256), static_cast<uint32_t>(smem), s,
                      at<qkv_v4i>(ws, L.aq), at<float>(ws, L.rowc), a.M, a.kst, a.norms, a.N,
                      nsplit, vlen, n_items, a.k, at<float>(ws, L.cs), at<int>(ws, L.ci),
-                     at<uint32_t>(ws, L.gth), over, cap);
+                     at<uint32_t>(ws, L.gth), left);
   QKV_LAUNCHED();
   const int64_t msmem = int64_t(nsplit) * a.k * 8;
   if (msmem > 65536)
@@ -1209,20 +1303,24 @@ int launch_passes(const MipsArgs& a, void* ws, const MipsLayout& L, const MipsPl
   float* mx = at<float>(ws, L.mx);
   hipLaunchKernelGGL((mips_pass<MB, PDW, QT, false>), grid, dim3(256), 0, s,
                      at<qkv_v4i>(ws, L.af), at<int>(ws, L.cil), thr, a.kst, a.norms, a.N,
-                     pl.ntile, pl.wq, pl.pb, ng1, pl.step, ft, mx, cnt, at<int>(ws, L.cand),
+                     pl.ntile, pl.wq, pl.pb, ng1, pl.step, a.M, ft, mx, cnt, at<int>(ws, L.cand),
                      pl.cap);
   QKV_LAUNCHED();
   const unsigned mq = static_cast<unsigned>(pl.ntile * QT * 16);
+  const float* unit = at<float>(ws, L.unit);
+  uint32_t* gth = at<uint32_t>(ws, L.gth);
   if (a.k <= 16)
-    hipLaunchKernelGGL(mips_bound<1>, dim3(mq), dim3(256), 0, s, mx, 16 * pl.P, a.k, a.M, thr, cnt,
-                       pl.cap);
+    hipLaunchKernelGGL(mips_bound<1>, dim3(mq), dim3(256), 0, s, mx, 16 * pl.P, a.k, a.M, pl.step,
+                       unit, at<int>(ws, L.ciu), at<int>(ws, L.cil), a.norms, a.N, thr, cnt,
+                       pl.cap, gth);
   else
-    hipLaunchKernelGGL(mips_bound<4>, dim3(mq), dim3(256), 0, s, mx, 16 * pl.P, a.k, a.M, thr,
-                       cnt, pl.cap);
+    hipLaunchKernelGGL(mips_bound<4>, dim3(mq), dim3(256), 0, s, mx, 16 * pl.P, a.k, a.M, pl.step,
+                       unit, at<int>(ws, L.ciu), at<int>(ws, L.cil), a.norms, a.N, thr, cnt,
+                       pl.cap, gth);
   QKV_LAUNCHED();
   hipLaunchKernelGGL((mips_pass<MB, PDW, QT, true>), grid, dim3(256), 0, s,
                      at<qkv_v4i>(ws, L.af), at<int>(ws, L.ciu), thr, a.kst, a.norms, a.N,
-                     pl.ntile, pl.wq, pl.pb, ng, 1, ft, mx, cnt, at<int>(ws, L.cand), pl.cap);
+                     pl.ntile, pl.wq, pl.pb, ng, 1, a.M, ft, mx, cnt, at<int>(ws, L.cand), pl.cap);
   QKV_LAUNCHED();
   return QKV_OK;
 }
@@ -1233,7 +1331,8 @@ int launch_filter(const MipsArgs& a, void* ws, const MipsLayout& L, const MipsPl
   int* cnt = at<int>(ws, L.cnt);
   hipLaunchKernelGGL((mips_fprep<PDW>), dim3(static_cast<unsigned>(pl.ntile * pl.qt)),
                      dim3(256), 0, s, at<float>(ws, L.qw), at<float>(ws, L.rowc), a.M, ft,
-                     at<uint32_t>(ws, L.af), at<int>(ws, L.ciu), at<int>(ws, L.cil), cnt, pl.cap);
+                     at<uint32_t>(ws, L.af), at<int>(ws, L.ciu), at<int>(ws, L.cil), cnt, pl.cap,
+                     at<float>(ws, L.unit), at<int>(ws, L.left), at<int>(ws, L.claimed));
   QKV_LAUNCHED();
   int st;
   switch (pl.qt) {
@@ -1246,7 +1345,7 @@ int launch_filter(const MipsArgs& a, void* ws, const MipsLayout& L, const MipsPl
   hipLaunchKernelGGL((mips_pick<MB, PDW>), dim3(a.M), dim3(256),
                      static_cast<uint32_t>(pl.cap * 8), s, at<qkv_v4i>(ws, L.aq),
                      at<float>(ws, L.rowc), a.kst, a.norms, a.k, cnt, at<int>(ws, L.cand), pl.cap,
-                     a.out_s, a.out_i);
+                     at<int>(ws, L.left), at<int>(ws, L.claimed), a.out_s, a.out_i);
   QKV_LAUNCHED();
   return QKV_OK;
 }
@@ -1296,8 +1395,8 @@ int mips_batch(const MipsArgs& a, void* ws, const Tables& tb, hipStream_t s) {
       const int st = launch_filter<MBV, PDWV>(a, ws, L, pl, ft, s);                        \
       if (st != QKV_OK) return st;                                                         \
     }                                                                                      \
-    return launch_scan<MBV, PDWV>(a, ws, L, nsplit, pl.filt ? at<int>(ws, L.cnt) : nullptr, \
-                                  pl.cap, s);
+    return launch_scan<MBV, PDWV>(a, ws, L, nsplit, pl.filt ? at<int>(ws, L.left) : nullptr, \
+                                  pl.filt ? at<int>(ws, L.cnt) : nullptr, pl.cap, s);
     QKV_MIPS(1, 2) QKV_MIPS(1, 3) QKV_MIPS(1, 4)
     QKV_MIPS(2, 2) QKV_MIPS(2, 3) QKV_MIPS(2, 4)
     QKV_MIPS(3, 2) QKV_MIPS(3, 3) QKV_MIPS(3, 4)

@@ -106,3 +106,26 @@ def test_large_signs(size):
     idx.add(torch.randn(30000, 128, device=DEV, generator=g))
     idx.quantizer.S = idx.quantizer.S * size
     _same(idx, torch.randn(40, 128, device=DEV, generator=g), 10)
+
+
+@pytest.mark.parametrize("d,n,m,copies,k", [
+    (128, 60000, 203, 2000, 10),   # predicted from the sampled groups: never listed
+    (128, 60000, 37, 1100, 10),    # past the cap by little: found while listing
+    (64, 60000, 301, 5000, 64), (128, 6000, 70, 1500, 3), (96, 40000, 1, 3000, 10),
+    (128, 60000, 513, 30000, 10),  # half of the vectors equal
+])
+def test_some_queries_left_to_the_full_scan(d, n, m, copies, k):
+    """Queries of duplicated vectors among others: the full scan takes their 4-query
+    chunks alone and starts from the filter's bound."""
+    g = torch.Generator(device=DEV).manual_seed(n + m)
+    db = torch.randn(n, d, device=DEV, generator=g)
+    q = torch.randn(m, d, device=DEV, generator=g)
+    hit = torch.randperm(m, device=DEV, generator=g)[: max(1, m // 20)]
+    for i, j in enumerate(hit[: max(1, n // (2 * copies))].tolist()):
+        at = torch.randperm(n, device=DEV, generator=g)[:copies]
+        db[at] = 2.0 * q[j]
+    idx = QuashIndex(dim=d, bits=3, seed=3, device=DEV)
+    idx.add(db)
+    _same(idx, q, k)
+    _same(idx, q[hit].contiguous(), k)
+    _same(idx, -q, k)
