@@ -546,29 +546,47 @@ __global__ __launch_bounds__(kThr, 2) void prefill(PreArgs A, KVLayers kv) {
 
       // scores: rows tokens, this lane's column its query row
       v16f S = {};
-      auto qjl = [&](int kk) {
-        const v4u sa = *reinterpret_cast<const v4u*>(buf + kk * 1024 + lane * 16 + C::OFF_S);
-        // (opaque: as loop invariants wh and wl would take 64 registers and spill)
+      const uint8_t* const at = buf + lane * 16;
+      auto op = [&](int ofs, int kk) {
+        return *reinterpret_cast<const v4u*>(at + ofs + kk * 1024);
+      };
+      // |q~| = |hi| + lo sign(hi)  (opaque: as loop invariants the two would take 64
+      // registers and spill)
+      auto magnitudes = [&](int kk, v4u& wh, v4u& wl) {
         asm volatile("" : "+v"(qhi[kk]));
-        // |q~| = |hi| + lo sign(hi)
-        const v4u wh = qhi[kk] & 0x7fff7fffu, wl = qlo[kk] ^ (qhi[kk] & 0x80008000u);
-        S = mfma_h(sa, wh, S);
-        S = mfma_h(sa, wl, S);
+        wh = qhi[kk] & 0x7fff7fffu;
+        wl = qlo[kk] ^ (qhi[kk] & 0x80008000u);
       };
       if constexpr (C::AE) {  // the whole QJL term first, to mend its weight
 #pragma unroll
-        for (int kk = 0; kk < KK; ++kk) qjl(kk);
-        S *= 1.f + A.ae;
-      }
+        for (int kk = 0; kk < KK; ++kk) {
+          const v4u sa = op(C::OFF_S, kk);
+          v4u wh, wl;
+          magnitudes(kk, wh, wl);
+          S = mfma_h(sa, wh, S);
+          S = mfma_h(sa, wl, S);
+        }
+        // (as S (1 + ae) the schedule around it was 2.4 % slower)
 #pragma unroll
-      for (int kk = 0; kk < KK; ++kk) {
-        const uint8_t* at = buf + kk * 1024 + lane * 16;
-        const v4u ka = *reinterpret_cast<const v4u*>(at);
-        S = mfma_h(ka, qhi[kk], S);
-        if constexpr (!C::AE) qjl(kk);
-        S = mfma_h(ka, qlo[kk], S);
-        if constexpr (C::KLO)
-          S = mfma_h(*reinterpret_cast<const v4u*>(at + C::SEG), qhi[kk], S);
+        for (int r = 0; r < 16; ++r) S[r] = fmaf(S[r], A.ae, S[r]);
+#pragma unroll
+        for (int kk = 0; kk < KK; ++kk) {
+          const v4u ka = op(0, kk);
+          S = mfma_h(ka, qhi[kk], S);
+          S = mfma_h(ka, qlo[kk], S);
+        }
+      } else {
+#pragma unroll
+        for (int kk = 0; kk < KK; ++kk) {
+          const v4u ka = op(0, kk), sa = op(C::OFF_S, kk);
+          v4u wh, wl;
+          magnitudes(kk, wh, wl);
+          S = mfma_h(ka, qhi[kk], S);
+          S = mfma_h(sa, wh, S);
+          S = mfma_h(ka, qlo[kk], S);
+          S = mfma_h(sa, wl, S);
+          if constexpr (C::KLO) S = mfma_h(op(C::SEG, kk), qhi[kk], S);
+        }
       }
       if (third) {
 #pragma unroll 1
