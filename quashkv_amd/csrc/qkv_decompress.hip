@@ -363,7 +363,7 @@ template <int D, int R>
 __device__ __forceinline__ void mma_store(const uint4 (&ah)[R][Geo<D>::NK],
                                           const uint4 (&al)[R][Geo<D>::NK], const float (&nf)[R],
                                           const uint4* frag, int lane, uint8_t* ost,
-                                          __amdgpu_buffer_rsrc_t ob, int out_dtype) {
+                                          __amdgpu_buffer_rsrc_t ob, int out_dtype, bool stream) {
   constexpr int NK = Geo<D>::NK, NJ = Geo<D>::NJ;
   constexpr int NSTEP = (NJ / 2) * NK;
   const int m = lane & 15, g = lane >> 4;
@@ -437,15 +437,31 @@ __device__ __forceinline__ void mma_store(const uint4 (&ah)[R][Geo<D>::NK],
     // 16-byte chunks: cpr per row segment, 64 / cpr rows per store
     const int cpr = 2 * obytes, rows = 64 / cpr;
     const int q = lane % cpr;
-    for (int v = lane / cpr; v < 16 * R; v += rows) {
-      const uint4 w = *reinterpret_cast<const uint4*>(ost + v * rsb + 16 * q);
-      // non-temporal (aux 2): rows that fill whole lines and outgrow the caches;
-      // without it the write-backs share the L2 with the codes' reads (524,288 rows
-      // of K and of V, d = 128, fp32: 188 -> 159 us, and 195 -> 148 on another card)
-      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(qkv_u32x4, w), ob,
-                                             (v * D + 32 * p) * obytes + 16 * q, 0, 2);
+    auto chunk = [&](int v) {
+      return __builtin_bit_cast(qkv_u32x4, *reinterpret_cast<const uint4*>(ost + v * rsb + 16 * q));
+    };
+    if (stream) {  // non-temporal (aux 2)
+      for (int v = lane / cpr; v < 16 * R; v += rows)
+        __builtin_amdgcn_raw_buffer_store_b128(chunk(v), ob, (v * D + 32 * p) * obytes + 16 * q, 0,
+                                               2);
+    } else {
+      for (int v = lane / cpr; v < 16 * R; v += rows)
+        __builtin_amdgcn_raw_buffer_store_b128(chunk(v), ob, (v * D + 32 * p) * obytes + 16 * q, 0,
+                                               0);
     }
   }
+}
+
+// Whether a call's output rows bypass the caches (the last level holds 256 MiB): then
+// their write-backs do not share the L2 with the codes' reads (fp32, d = 128, 256 MiB:
+// 82.8 us, non-temporal 68.8; with a sum over the rows after it 165 and 161).  Smaller
+// outputs stay for the kernel that reads them: 98 MiB and a product 127 us,
+// non-temporal 138; 48 MiB 86 and 102 (146 MiB and a sum 182 and 184, alone 47 and
+// 46).  At d = 64 the line is higher: 98 MiB and a product 112 and 128, 195 MiB 252 and
+// 264, 256 MiB 224 and 225 (alone 73 and 58).
+template <int D>
+__device__ __forceinline__ bool bypass_caches(int64_t n, int obytes) {
+  return n * D * obytes >= int64_t(D == 128 ? 128 : 256) << 20;
 }
 
 // A block's place: group, first token, end of the group's valid tokens.
@@ -507,6 +523,7 @@ __global__ __launch_bounds__(kThreads, 2) void decompress_waves(
                    : FMT == QKV_FMT_KPLANES ? int64_t(bits + 1) * (D / 8) : D;
   const int64_t pq = FMT == QKV_FMT_PACKED ? D / 8 : D;
   const int obytes = out_dtype == QKV_F32 ? 4 : 2;
+  const bool stream = bypass_caches<D>(n, obytes);
   uint4* stg = &stage[wave * 288];
 
   Raw<D, FMT, BITS, IP, R> x;
@@ -604,7 +621,7 @@ __global__ __launch_bounds__(kThreads, 2) void decompress_waves(
     fetch(more ? nb : blk);  // unconditional: the last round re-reads its own block
     const BlockPos b(blk, bpg, RB, n, in_seq);
     mma_store<D, R>(ah, al, nf, frag, lane, reinterpret_cast<uint8_t*>(stg),
-                    out_rsrc(out, b, RB, D, obytes, in_seq), out_dtype);
+                    out_rsrc(out, b, RB, D, obytes, in_seq), out_dtype, stream);
     if (!more) break;
     expand_fetched();
     blk = nb;
@@ -743,6 +760,7 @@ __global__ __launch_bounds__(64 * (NC + 1), 1) void decompress_staged(
     LaneConsts<D, IP, SEL> lc;
     lc.load(g, sel, signs, qjl_scale, sv);
     const int obytes = out_dtype == QKV_F32 ? 4 : 2;
+    const bool stream = bypass_caches<D>(n, obytes);
     lds_barrier();
     for (int round = 0; round < rounds; ++round) {
       const int blk = block_of(round, wave);
@@ -786,7 +804,7 @@ __global__ __launch_bounds__(64 * (NC + 1), 1) void decompress_staged(
         for (int r = 0; r < R; ++r) nf[r] = x.n[r] * ofac;
         const BlockPos b(blk, bpg, RB, n, in_seq);
         mma_store<D, R>(ah, al, nf, frag, lane, const_cast<uint8_t*>(sl),
-                        out_rsrc(out, b, RB, D, obytes, in_seq), out_dtype);
+                        out_rsrc(out, b, RB, D, obytes, in_seq), out_dtype, stream);
       }
       lds_barrier();
     }

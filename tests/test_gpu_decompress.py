@@ -208,3 +208,17 @@ def test_decompress_cfg3_size_vs_float64_gemm():
             rel_den += float((ref * ref).sum())
     rel = (rel_num / rel_den) ** 0.5
     assert rel <= 3e-6 and worst <= 1e-5, (rel, worst)
+
+
+@pytest.mark.parametrize("d,n", [(128, 1 << 18), (64, 1 << 20), (96, (1 << 28) // 384 + 1)])
+def test_decompress_rows_past_the_caches(d, n):
+    """Outputs from the size at which the stores bypass the caches up: the same bits as
+    in parts that stay below it."""
+    g = torch.Generator(device="cuda").manual_seed(d)
+    q = Q.MSEQuantizer(d, 3, seed=5, device="cuda")
+    codes = torch.randint(0, 8, (n, d), device="cuda", generator=g).to(torch.uint8)
+    norms = torch.rand(n, device="cuda", generator=g) + 0.5
+    rows = q.decompress(codes, norms)
+    h = n // 2 + 5
+    assert torch.equal(rows[:h], q.decompress(codes[:h], norms[:h]))
+    assert torch.equal(rows[h:], q.decompress(codes[h:].contiguous(), norms[h:].contiguous()))
