@@ -1141,11 +1141,14 @@ int filt_batch(int k) { return 16384 * 1024 / filt_cap(k); }
 // The filter serves every k <= 64 (its bound comes from 1024 maxima at most):
 // a scan's lists fill at ~0.7 ms per call whatever the size (top-10 of 10^4
 // vectors for 64 queries 753 us, filtered 78; for one query 116 and 49; of 10^6
-// for 10^4 queries 13.1 ms and 3.0), so no smaller search is better off there
-// (N = 2048, one query: 113 and 49 us; k = 1, d = 96: 63 and 38).
+// for 10^4 queries 13.1 ms and 3.0).  One or two queries over a few hundred
+// vectors are the exception, where a scan is two launches against seven (top-1 of
+// 256: 24 - 29 us and 37 - 44; of 700: 34 - 45 and 38 - 44; top-3 of 400: 34 - 43
+// and 40 - 46; top-10 of 256: 50 - 60 and 38 - 51).
 MipsPlan mips_plan(int32_t M, int64_t N, int k) {
   MipsPlan pl{};
-  pl.filt = k <= kFiltKMax && N >= kFiltMinN;
+  const bool tiny = M <= 2 && N < 700 && N * N * k * M < 700 * 700;
+  pl.filt = k <= kFiltKMax && N >= kFiltMinN && !tiny;
   if (!pl.filt) return pl;
   pl.qt = M <= 16 ? 1 : M <= 64 ? 2 : M <= 1024 ? 4 : kFiltQT;
   pl.ntile = (M + 16 * pl.qt - 1) / (16 * pl.qt);

@@ -36,6 +36,8 @@ def _same(idx, q, k):
     (64, 3, 50016, 200, 10), (64, 4, 65599, 40, 32), (64, 2, 40001, 31, 5),
     (128, 3, 256, 5, 10), (64, 3, 300, 70, 64), (128, 4, 8191, 20, 64), (96, 2, 8192, 20, 9),
     (96, 3, 49999, 64, 10), (96, 4, 33333, 129, 10), (96, 2, 34567, 257, 3),
+    # either side of the line below which the scan runs
+    (128, 3, 699, 1, 1), (128, 3, 700, 1, 1), (64, 3, 350, 2, 2), (64, 3, 349, 2, 2),
 ])
 def test_filter_equals_full_scan(d, bits, n, m, k):
     g = torch.Generator(device=DEV).manual_seed(n + m)
@@ -45,7 +47,8 @@ def test_filter_equals_full_scan(d, bits, n, m, k):
     idx.add(db)
     q = torch.randn(m, d, device=DEV, generator=g)
     q[: m // 2] *= torch.logspace(-6, 6, m // 2, device=DEV)[:, None]
-    q[m // 3, 1:] = 0.0                                      # one coordinate only
+    if m > 2:
+        q[m // 3, 1:] = 0.0                                  # one coordinate only
     _same(idx, q, k)
 
 
