@@ -305,10 +305,13 @@ __global__ __launch_bounds__(kThr, 2) void prefill(PreArgs A, KVLayers kv) {
           x[i >> 3][i & 7] = static_cast<float>(__builtin_bit_cast(
               _Float16, static_cast<uint16_t>(raw[i >> 3][(i & 7) >> 1] >> (16 * (i & 1)))));
       }
-    } else {
-#pragma unroll
+    } else {  // (rolled, through LDS: unrolled it was near half of the kernel's code)
+      float* const t = reinterpret_cast<float*>(lds + 2 * C::IMG + wave * C::OPND) + lane;
+#pragma unroll 1
       for (int i = 0; i < 8 * KK; ++i)
-        x[i >> 3][i & 7] = qkv_load(A.q, q0 + 16 * (i >> 3) + (i & 7), A.q_dtype);
+        t[64 * i] = qkv_load(A.q, q0 + 16 * (i >> 3) + (i & 7), A.q_dtype);
+#pragma unroll
+      for (int i = 0; i < 8 * KK; ++i) x[i >> 3][i & 7] = t[64 * i];
     }
     stage_pi<CT, false>(A.pi, lds, tid);
     float amax = 0.f;

@@ -354,3 +354,15 @@ def test_prefill_precision(d, kb, vb, scale, bar):
     q = scale * torch.randn(4, 32, 64, d, device=DEV, generator=g)
     assert prefills(e, q)
     check(e.attention(q, causal=True), exact(e, q, True), bar)
+
+
+@pytest.mark.parametrize("d,dtype", [(128, torch.float32), (128, torch.bfloat16),
+                                     (96, torch.float16), (64, torch.float32)])
+def test_prefill_unaligned_queries(d, dtype):
+    e, g = filled(8, 8, 200, d, 3, 3, 37)
+    n = 8 * 32 * 80 * d
+    q = torch.randn(n + 1, device=DEV, generator=g).to(dtype)[1:].view(8, 32, 80, d)
+    assert prefills(e, q) and q.is_contiguous() and q.data_ptr() % 16
+    out = e.attention(q, causal=True)
+    assert torch.equal(out, e.attention(q.clone(), causal=True))
+    check(out, exact(e, q, True))
