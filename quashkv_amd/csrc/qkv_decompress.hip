@@ -452,16 +452,19 @@ __device__ __forceinline__ void mma_store(const uint4 (&ah)[R][Geo<D>::NK],
   }
 }
 
-// Whether a call's output rows bypass the caches (the last level holds 256 MiB): then
-// their write-backs do not share the L2 with the codes' reads (fp32, d = 128, 256 MiB:
-// 82.8 us, non-temporal 68.8; with a sum over the rows after it 165 and 161).  Smaller
-// outputs stay for the kernel that reads them: 98 MiB and a product 127 us,
-// non-temporal 138; 48 MiB 86 and 102 (146 MiB and a sum 182 and 184, alone 47 and
-// 46).  At d = 64 the line is higher: 98 MiB and a product 112 and 128, 195 MiB 252 and
-// 264, 256 MiB 224 and 225 (alone 73 and 58).
+// Whether a call's output rows bypass the caches.  Past about half of the 256 MiB last
+// level: their write-backs then do not share the L2 with the codes' reads (fp32, d =
+// 128, 256 MiB: 82.8 us, non-temporal 68.8; with a sum over the rows after it 165 and
+// 161).  Between, the rows stay for the kernel that reads them: 98 MiB and a product
+// 122 us, non-temporal 132; 48 MiB 86 and 100, though alone 27 and 21 (146 MiB and a
+// product 285 and 283).  At most the L2s' 32 MiB at d = 128: 15 MiB and a sum 27.5 us,
+// non-temporal 22.9; 31 MiB 33.5 and 32.7.  At d = 64 15 MiB is the same either way and
+// the upper line higher: 195 MiB and a product 252 and 264, 256 MiB 224 and 225 (alone
+// 73 and 58).
 template <int D>
 __device__ __forceinline__ bool bypass_caches(int64_t n, int obytes) {
-  return n * D * obytes >= int64_t(D == 128 ? 128 : 256) << 20;
+  const int64_t mib = (n * D * obytes) >> 20;
+  return D == 128 ? mib < 32 || mib >= 128 : mib >= 256;
 }
 
 // A block's place: group, first token, end of the group's valid tokens.

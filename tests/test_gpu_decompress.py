@@ -210,10 +210,11 @@ def test_decompress_cfg3_size_vs_float64_gemm():
     assert rel <= 3e-6 and worst <= 1e-5, (rel, worst)
 
 
-@pytest.mark.parametrize("d,n", [(128, 1 << 18), (64, 1 << 20), (96, (1 << 28) // 384 + 1)])
+@pytest.mark.parametrize("d,n", [(128, 1 << 18), (64, 1 << 20), (96, (1 << 28) // 384 + 1),
+                                 (128, 1 << 16)])
 def test_decompress_rows_past_the_caches(d, n):
-    """Outputs from the size at which the stores bypass the caches up: the same bits as
-    in parts that stay below it."""
+    """Outputs of sizes where the stores begin or cease to bypass the caches: the same
+    bits as in two parts, on the other side of the line."""
     g = torch.Generator(device="cuda").manual_seed(d)
     q = Q.MSEQuantizer(d, 3, seed=5, device="cuda")
     codes = torch.randint(0, 8, (n, d), device="cuda", generator=g).to(torch.uint8)
