@@ -302,12 +302,15 @@ int qkv_vtiles_unpack(const uint32_t* src, int64_t groups, int64_t S, int32_t d,
  *   t_stride   token capacity (multiple of 32; 64 for the MFMA path)
  *   T          valid tokens (<= t_stride); causal masks kv_pos > T - Q + i
  *   kcent_host, vcent_host  HOST arrays of the 2^kbits / 2^vbits centroids
- *   signs      d fp32, the QJL sign vector S: +-1 (other magnitudes within
- *              1e-3 .. 1e3 of each other and of 1 are served as they are)
+ *   signs      d fp32, the QJL sign vector S: +-1 (other magnitudes of that
+ *              order are served as they are)
  *   out        B x Hq x Q x d, out_dtype
  *   workspace  >= qkv_attention_workspace_bytes(..., n_splits), 256-B aligned
- * Symmetric codebooks (all Lloyd-Max codebooks are) with d = 128 and
- * kbits <= 2 run on the integer-MFMA kernel; other shapes on a VALU kernel.
+ * Symmetric codebooks (all Lloyd-Max codebooks are) with kbits <= 3, d = 64, 96
+ * or 128 and t_stride a multiple of 64 run on MFMA kernels: decode_fused, at d =
+ * 64 with kbits <= 2 and no key ranges decode_small, and with 48 or more query
+ * rows per kv head, where it is faster, prefill (qkv_attention_prefills).  Other
+ * codebooks and strides run on a VALU kernel.
  * ---------------------------------------------------------------------- */
 
 /* Split-K count the library would use for a decode-attention call.  (A call of

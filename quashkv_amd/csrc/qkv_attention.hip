@@ -2249,7 +2249,7 @@ static int32_t decode_splits(int32_t B, int32_t Hq, int32_t Hkv, int32_t Q, int3
 // ps of its own: both kernels' times in us as measured (rounds of the chip's
 // workgroups times their steps; fixed part; the merge of splits).  E.g. d = 128, 8
 // groups: 48 rows over 256 keys 19 against 28 us, over 8192 keys 51 against 37; 256
-// rows over 2048 keys 42 against 39; 8192 rows over 2048 keys 1052 against 155.
+// rows over 2048 keys 42 against 39; 8192 rows over 2048 keys 1056 against 142.
 // small: decode_small serves the call (d = 64, key MSE bits <= 2, no key ranges); at
 // d = 64 decode_fused is a good deal slower (96 groups of 287 rows over 95 keys: 56 us
 // in decode_small, 301 in decode_fused with 2 key MSE bits, 413 with 3; 27 here).

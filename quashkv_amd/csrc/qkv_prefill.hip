@@ -38,13 +38,16 @@
 // keys and values; beside them ~250 VALU instructions of softmax and ~140 of
 // expansion per wave.  One workgroup per CU (LDS: two 64-token buffers); of the two
 // waves on a SIMD one expands before its products and the other after.  Measured,
-// Q = T = 2048, 32 query and 8 kv heads, d = 128, causal: 141 us against 1056 us on
-// the decode kernel (matrix cores busy 38 %); 4.4 us per 64-token step.  On the
-// way: 4 waves per workgroup, two workgroups per CU 447 us; 8 waves 284; q~'s |.|
-// parts kept out of loop-invariant registers (spills, whose reloads wait for the
-// loads in flight) 244; the halves' phases staggered 230; two QJL products instead
-// of three 160; set-up loads issued together and its tiles shared by the wave
-// pairs 144.  A second accumulator chain for the QJL products changed nothing.
+// Q = T = 2048, 32 query and 8 kv heads, d = 128, causal, a pass among others: 142 -
+// 151 us on three cards against 1056 - 1064 us on the decode kernel (164 - 167 us with
+// a wait after each; matrix cores busy 37 %); 4.4 us per 64-token step.  On the way:
+// 4 waves per workgroup, two workgroups per CU 447 us; 8 waves 284; q~'s |.| parts
+// kept out of loop-invariant registers (spills, whose reloads wait for the loads in
+// flight) 244; the halves' phases staggered 230; two QJL products instead of three
+// 160; set-up loads issued together and its tiles shared by the wave pairs 140; f16
+// pairs rounded to nearest and the QJL weight mended 142.  2-bit values: hi + lo
+// levels 142 - 147 us, one f16 each 133.  A second accumulator chain for the QJL
+// products changed nothing.
 #include <math.h>
 
 #include <algorithm>
