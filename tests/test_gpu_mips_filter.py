@@ -132,3 +132,29 @@ def test_some_queries_left_to_the_full_scan(d, n, m, copies, k):
     _same(idx, q, k)
     _same(idx, q[hit].contiguous(), k)
     _same(idx, -q, k)
+
+
+def test_replays_of_a_captured_search():
+    """The list of chunks left to the full scan is the replay's own: queries change
+    between replays from ones that overflow to ones that do not, and back."""
+    g = torch.Generator(device=DEV).manual_seed(9)
+    db = torch.randn(30000, 128, device=DEV, generator=g)
+    hot = torch.randn(3, 128, device=DEV, generator=g)
+    db[:4000] = hot[0]
+    idx = QuashIndex(dim=128, bits=3, seed=3, device=DEV)
+    idx.add(db)
+    plain = torch.randn(50, 128, device=DEV, generator=g)
+    mixed = plain.clone()
+    mixed[[0, 17, 49]] = hot[0]
+    q = mixed.clone()
+    idx.search(q, 10)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        s, i = idx.search(q, 10)
+    for new in (mixed, plain, mixed, plain):
+        q.copy_(new)
+        graph.replay()
+        torch.cuda.synchronize()
+        got_s, got_i = s.clone(), i.clone()
+        es, ei = idx.search(q, 10)
+        assert torch.equal(got_i, ei) and torch.equal(got_s, es)
